@@ -747,331 +747,7 @@ void launch_attn_hpg(const AttnLaunch& a, hipStream_t st) {
   }
 }
 
-// ---------------------------------------------------------------------------------------------------------------
-// Prefill attention: causal attention of M prompt rows (row m at position pos + m) over the paged cache, which already
-// holds their K / V. A workgroup owns one kv head and QB = 64 / HPG consecutive rows, and runs KVS groups of four
-// waves. Wave w of every group has the same 16 MFMA columns, (row, query head) pairs, PW = 16 / HPG rows x HPG heads,
-// so every column does work; group h takes the 64-token blocks b with b % KVS == h. The K / V of the tokens
-// [0, last row's position] stream through LDS in rounds of KVS blocks (double-buffered, the next rounds' loads in
-// flight in registers during the current round's MFMAs), one block per group, read there by the group's four waves.
-// With KVS = 2, two waves share each SIMD and each works through half the blocks: the launcher takes it when the grid
-// leaves CUs with one workgroup or none, where a lone wave per SIMD waits on its own per-block chain (about 430 vector
-// instructions around 48 MFMAs); with more workgroups than CUs the grid fills the SIMDs by itself (KVS = 1).
-// Per 16-token tile the math is the MFMA decode kernel's: S^T = K . Q^T (the accumulator is P's A operand as is), the
-// causal bound of each column applied to its own scores, online softmax once per block, P . V with p as fp16 hi + lo
-// parts and V operands built by byte permutes from 4 token rows. The groups' states (running max, sum, accumulator per
-// column) meet in LDS at the end and group 0 merges them in group order. Every column's tokens go to the same group in
-// the same order whatever workgroup or batch its row is in (block b to group b % KVS, from token 0), and a block
-// wholly past a column's bound changes nothing for it, so a row's result does not depend on how the prompt is
-// batched; for a given KVS. The launch's KVS depends on the grid, so the split of a prompt into launches can change it.
-constexpr int kPfGroupWaves = 4, kPfBlock = 64, kPfPages = 2048, kPfRing = 2;
-// Running maximum of a column that has seen no token yet: a finite stand-in for -infinity, so that exp(max_old -
-// max_new) and exp(score - max) never meet -inf - (-inf); exp(-1e30 - x) is 0 for every score x.
-constexpr float kPfNoMax = -1e30f;
-
-// Keeps loads where they are written (no sinking to their first use; see the K / V ring below).
-__device__ __forceinline__ void pf_fence() { asm volatile("" ::: "memory"); }
-
-template <int D, int HPG, int KVS>
-__global__ void __launch_bounds__(kPfGroupWaves * kWave * KVS)
-attn_prefill_kernel(const f16* __restrict__ qkv, const int32_t* __restrict__ pos_ptr, const int32_t* __restrict__ bt,
-                    int n_bt, const f16* kc, const f16* vc, int n_pages, int log2P, int n_q, int n_kv, int M,
-                    int ctx_cap, float scale, f16* __restrict__ out) {
-  // (kc, vc without __restrict__: the fences must order their loads)
-  using S = MfmaAttnShape<D>;
-  constexpr int KD = S::KD, KW = S::KW, QS = S::QS, VD = S::VD;
-  constexpr int NTH = kPfGroupWaves * kWave * KVS;       // threads
-  constexpr int PW = 16 / HPG;                           // rows per wave
-  constexpr int QB = kPfGroupWaves * PW;                 // rows per workgroup
-  constexpr int ROW = D + 8;                             // padded LDS row: 16 rows of one K read in distinct banks
-  constexpr int CH = D / 8;                              // 16-byte chunks per K / V row
-  constexpr int SB = kPfBlock * KVS;                     // tokens per round (one block per group)
-  constexpr int LPT = SB * CH / NTH;                     // 16-byte K (and V) loads per thread per round
-  constexpr int RPI = NTH / CH;                          // token rows covered per load index
-  __shared__ __align__(16) f16 Ks[2][SB][ROW];
-  __shared__ __align__(16) f16 Vs[2][SB][ROW];
-  __shared__ int s_pg[kPfPages];
-
-  const int kvh = blockIdx.x, qb = blockIdx.y;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int grp = wave / kPfGroupWaves, gw = wave % kPfGroupWaves;  // group, and the wave's columns within it
-  const int col = lane & 15, g = lane >> 4;
-  const int P = 1 << log2P;
-  const int pos0 = *pos_ptr;
-  // this lane's query column: prompt row m, head h; tokens t <= lim are attended
-  const int mw = qb * QB + gw * PW;                      // the wave's first row
-  const int m = mw + col / HPG;
-  const int h = kvh * HPG + col % HPG;
-  const bool live = m < M;
-  const int lim = live ? min(pos0 + m, ctx_cap - 1) : -1;  // the cap bounds the mask as well as the loads
-  const int mlast = min(qb * QB + QB, M) - 1;
-  const int ctx = (int)max(0LL, min((long long)pos0 + mlast + 1, (long long)ctx_cap));  // tokens [0, ctx) are read
-  const int npg = (ctx + P - 1) >> log2P;
-  const bool staged = npg <= kPfPages;  // uniform: block-table pages in LDS, else read per token from global
-  if (staged)
-    for (int i = tid; i < npg; i += NTH) s_pg[i] = bt[i];
-  u32x4 qr[KW];
-  {
-    const f16* qh = qkv + (size_t)(live ? m : 0) * (n_q + 2 * n_kv) * D + (size_t)h * D;
-#pragma unroll
-    for (int w = 0; w < KW; ++w)
-      qr[w] = live ? *reinterpret_cast<const u32x4*>(qh + KD * g + 8 * w) : u32x4{0u, 0u, 0u, 0u};
-  }
-  __syncthreads();  // s_pg
-
-  // K / V ring: round r's loads go into register slot r % kPfRing kPfRing rounds before the round is computed and are
-  // staged into LDS buffer r & 1 one round before. Thread: chunk tid % CH of token rows tid / CH + RPI i of the round;
-  // tokens past ctx or without a page read page 0's row (every cache has one) and are zeroed by select.
-  const int nrnd = (ctx + SB - 1) / SB;
-  u32x4 kk[kPfRing][LPT], vv[kPfRing][LPT];
-  bool ok[kPfRing][LPT];
-  auto fetch = [&](int rnd, int slot) {
-    const int b0 = min(rnd, nrnd - 1) * SB;  // past the end: a re-read of the last round, never staged
-#pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const int t = b0 + tid / CH + RPI * i;
-      const int lp = t >> log2P;
-      int pg = t < ctx ? (staged ? s_pg[lp] : bt[lp]) : -1;
-      if (pg >= n_pages) pg = -1;
-      const size_t off =
-          ((((size_t)(pg < 0 ? 0 : pg) * n_kv + kvh) << log2P) + (t & (P - 1))) * D + 8 * (tid % CH);
-      kk[slot][i] = load_stream(reinterpret_cast<const u32x4*>(kc + off));
-      vv[slot][i] = load_stream(reinterpret_cast<const u32x4*>(vc + off));
-      ok[slot][i] = pg >= 0;
-    }
-  };
-  auto stage = [&](int buf, int slot) {
-    const u32x4 z = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int i = 0; i < LPT; ++i) {
-      const int r = tid / CH + RPI * i;
-      *reinterpret_cast<u32x4*>(&Ks[buf][r][8 * (tid % CH)]) = ok[slot][i] ? kk[slot][i] : z;
-      *reinterpret_cast<u32x4*>(&Vs[buf][r][8 * (tid % CH)]) = ok[slot][i] ? vv[slot][i] : z;
-    }
-  };
-
-  float mrun = kPfNoMax, l = 0.f;
-  f4 acc[VD];
-#pragma unroll
-  for (int t = 0; t < VD; ++t) acc[t] = f4{0.f, 0.f, 0.f, 0.f};
-
-  // the group's block of round rnd (tokens t0 .. t0 + 63, LDS rows r0 .. r0 + 63 of buffer buf)
-  auto compute = [&](int t0, int buf) {
-    const int r0 = grp * kPfBlock;
-    // ---- scores of the block's four 16-token tiles: sc[tt][v] = score of token 16 tt + 4 g + v for column col
-    f4 sc[4];
-    float rmax = -INFINITY;
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      u32x4 kr[KW];
-#pragma unroll
-      for (int w = 0; w < KW; ++w)
-        kr[w] = *reinterpret_cast<const u32x4*>(&Ks[buf][r0 + 16 * tt + col][KD * g + 8 * w]);
-      f4 c = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int q = 0; q < QS; ++q) {
-        const int i0 = 2 * q, i1 = 2 * q + 1;
-        c = mfma16(as_h4(kr[i0 >> 2][i0 & 3], kr[i1 >> 2][i1 & 3]), as_h4(qr[i0 >> 2][i0 & 3], qr[i1 >> 2][i1 & 3]),
-                   c);
-      }
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int t = t0 + 16 * tt + 4 * g + v;
-        sc[tt][v] = t <= lim ? c[v] * scale : -INFINITY;
-        rmax = fmaxf(rmax, sc[tt][v]);
-      }
-    }
-    // ---- online softmax, once per block (mrun is finite, so is mn: a masked score gives exp(-inf) = 0)
-    rmax = rows_max(rmax);
-    const float mn = fmaxf(mrun, rmax);
-    const float alpha = __expf(mrun - mn);
-    float ps = 0.f;
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const float pv = __expf(sc[tt][v] - mn);
-        sc[tt][v] = pv;
-        ps += pv;
-      }
-    }
-    l = alpha * l + rows_sum(ps);
-    mrun = mn;
-    // the accumulator's rows are columns 4 g + v: their rescale factors live in lanes 4 g + v
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const float av = __shfl(alpha, 4 * g + v, kWave);
-#pragma unroll
-      for (int t = 0; t < VD; ++t) acc[t][v] *= av;
-    }
-    // ---- P . V: p as fp16 hi + lo parts; V rows 16 tt + 4 g + v, dims VD col .. VD col + VD - 1
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-      h4 phi, plo;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        phi[v] = (f16)sc[tt][v];
-        plo[v] = (f16)(sc[tt][v] - (float)phi[v]);
-      }
-      VRow<VD> vr[4];
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const f16* src = &Vs[buf][r0 + 16 * tt + 4 * g + v][VD * col];
-        if constexpr (VD == 4) {
-          const u32x2 x = *reinterpret_cast<const u32x2*>(src);
-          vr[v].w[0] = x.x;
-          vr[v].w[1] = x.y;
-        } else {
-          const u32x4 x = *reinterpret_cast<const u32x4*>(src);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) vr[v].w[i] = x[i];
-        }
-      }
-#pragma unroll
-      for (int t = 0; t < VD; ++t) {
-        const int wi = t >> 1;
-        const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;
-        const uint32_t lo = __builtin_amdgcn_perm(vr[1].w[wi], vr[0].w[wi], sel);
-        const uint32_t hi = __builtin_amdgcn_perm(vr[3].w[wi], vr[2].w[wi], sel);
-        const h4 vb = as_h4(lo, hi);
-        acc[t] = mfma16(phi, vb, acc[t]);
-        acc[t] = mfma16(plo, vb, acc[t]);
-      }
-    }
-  };
-  // round rnd (u = rnd % kPfRing, a constant wherever this is called): the group's block from LDS buffer rnd & 1, stage
-  // round rnd + 1 from its slot into the other buffer (every wave finished reading it before the last barrier), refill
-  // that slot with round rnd + 1 + kPfRing. (Branching around the compute of blocks past the wave's rows, or around the
-  // rescale when no maximum moved, measured slower: up to 1.6x at head dim 128.)
-  auto step = [&](int rnd, int u) {
-    compute((rnd * KVS + grp) * kPfBlock, rnd & 1);
-    const int ns = (u + 1) % kPfRing;
-    stage((rnd + 1) & 1, ns);  // past the end: a stale slot into an unread buffer
-    pf_fence();
-    fetch(rnd + 1 + kPfRing, ns);
-    pf_fence();
-    __syncthreads();
-  };
-  if (nrnd > 0) {  // uniform
-#pragma unroll
-    for (int u = 0; u < kPfRing; ++u) {
-      fetch(u, u);
-      pf_fence();
-    }
-    stage(0, 0);
-    pf_fence();
-    fetch(kPfRing, 0);
-    pf_fence();
-    __syncthreads();
-    // whole groups of kPfRing rounds in the loop, the remainder after it (no exit between a group's rounds, which
-    // would leave a path where another slot's loads are the newest and the in-order waits drain everything)
-    int r0 = 0;
-    for (; r0 + kPfRing <= nrnd; r0 += kPfRing) {
-#pragma unroll
-      for (int u = 0; u < kPfRing; ++u) step(r0 + u, u);
-    }
-#pragma unroll
-    for (int u = 0; u + 1 < kPfRing; ++u)
-      if (r0 + u < nrnd) step(r0 + u, u);
-  }
-  // ---- merge: groups 1 .. KVS - 1 leave max and sum per column and the accumulator per lane in LDS (over the K / V
-  // buffers, which every wave has finished reading at the last barrier); group 0 merges them in group order
-  static_assert(KVS == 1 || (2 * KVS * kPfGroupWaves * 16 + (KVS - 1) * kPfGroupWaves * kWave * 4 * VD) * 4 <=
-                                (int)sizeof(Ks), "merge scratch fits the K buffers");
-  float* s_ml = reinterpret_cast<float*>(&Ks[0][0][0]);          // [2][KVS][waves][16]: max, then sum
-  float* s_acc = s_ml + 2 * KVS * kPfGroupWaves * 16;           // [KVS - 1][waves][lanes][VD][4]
-  if constexpr (KVS > 1) {
-    if (g == 0) {
-      s_ml[(grp * kPfGroupWaves + gw) * 16 + col] = mrun;
-      s_ml[((KVS + grp) * kPfGroupWaves + gw) * 16 + col] = l;
-    }
-    if (grp > 0) {
-      f4* dst = reinterpret_cast<f4*>(s_acc) + (((grp - 1) * kPfGroupWaves + gw) * kWave + lane) * VD;
-#pragma unroll
-      for (int t = 0; t < VD; ++t) dst[t] = acc[t];
-    }
-    __syncthreads();
-    if (grp > 0) return;  // uniform per wave; no barrier follows
-  }
-  // ---- output: acc[t][v] = O[column 4 g + v][dim VD col + t]
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int cc = 4 * g + v;
-    float inv;
-    if constexpr (KVS == 1) {
-      const float lv = __shfl(l, cc, kWave);  // the column's sum lives in lane 4 g + v
-      inv = lv > 0.f ? 1.0f / lv : 0.f;
-    } else {
-      float mx = kPfNoMax;
-#pragma unroll
-      for (int hh = 0; hh < KVS; ++hh) mx = fmaxf(mx, s_ml[(hh * kPfGroupWaves + gw) * 16 + cc]);
-      float wg[KVS], tot = 0.f;  // group hh's weight exp(m_hh - max) (0 for a group that saw no token)
-#pragma unroll
-      for (int hh = 0; hh < KVS; ++hh) {
-        wg[hh] = __expf(s_ml[(hh * kPfGroupWaves + gw) * 16 + cc] - mx);
-        tot = fmaf(wg[hh], s_ml[((KVS + hh) * kPfGroupWaves + gw) * 16 + cc], tot);
-      }
-      inv = tot > 0.f ? 1.0f / tot : 0.f;
-#pragma unroll
-      for (int t = 0; t < VD; ++t) {
-        float o = wg[0] * acc[t][v];
-#pragma unroll
-        for (int hh = 1; hh < KVS; ++hh)
-          o = fmaf(wg[hh], s_acc[((((hh - 1) * kPfGroupWaves + gw) * kWave + lane) * VD + t) * 4 + v], o);
-        acc[t][v] = o;
-      }
-    }
-    const int mm = mw + cc / HPG, hh = kvh * HPG + cc % HPG;
-    if (mm < M) {
-      f16* dst = out + (size_t)mm * n_q * D + (size_t)hh * D + VD * col;
-#pragma unroll
-      for (int t = 0; t < VD; ++t) dst[t] = (f16)(acc[t][v] * inv);
-    }
-  }
-}
-
-// Grids of at most this many workgroups (one round of the 256 CUs) run two wave groups per workgroup (KVS = 2).
-constexpr int kPfSplitGrid = 256;
-
-template <int D>
-void launch_prefill_hpg(const void* qkv, const int32_t* pos, const int32_t* bt, int n_bt, const void* kc,
-                        const void* vc, int n_pages, int log2P, int n_q, int n_kv, int M, int max_ctx, void* out,
-                        hipStream_t st) {
-  const float scale = 1.0f / sqrtf((float)D);
-  const int cap = (int)min((long long)max_ctx, (long long)n_bt << log2P);
-#define DK_PREFILL_KVS(H, KVS)                                                                                      \
-  hipLaunchKernelGGL((attn_prefill_kernel<D, H, KVS>), dim3(n_kv, rb), dim3(kPfGroupWaves * kWave * KVS), 0, st,  \
-                     (const f16*)qkv, pos, bt, n_bt, (const f16*)kc, (const f16*)vc, n_pages, log2P, n_q, n_kv, M, cap, \
-                     scale, (f16*)out)
-#define DK_PREFILL(H)                                                                                               \
-  {                                                                                                                 \
-    const int rb = (M + kPfGroupWaves * (16 / H) - 1) / (kPfGroupWaves * (16 / H));                                 \
-    if ((long long)n_kv * rb <= kPfSplitGrid)                                                                       \
-      DK_PREFILL_KVS(H, 2);                                                                                         \
-    else                                                                                                            \
-      DK_PREFILL_KVS(H, 1);                                                                                         \
-  }
-  switch (n_q / n_kv) {
-    case 1: DK_PREFILL(1); break;
-    case 2: DK_PREFILL(2); break;
-    case 4: DK_PREFILL(4); break;
-    default: DK_PREFILL(8); break;
-  }
-#undef DK_PREFILL
-#undef DK_PREFILL_KVS
-}
-
 }  // namespace
-
-void launch_attention_prefill(const void* qkv, const int32_t* pos, const int32_t* bt, int n_bt, const void* kc,
-                              const void* vc, int n_pages, int log2P, int n_q, int n_kv, int head_dim, int M,
-                              int max_ctx, void* out, hipStream_t st) {
-  if (head_dim == 64)
-    launch_prefill_hpg<64>(qkv, pos, bt, n_bt, kc, vc, n_pages, log2P, n_q, n_kv, M, max_ctx, out, st);
-  else
-    launch_prefill_hpg<128>(qkv, pos, bt, n_bt, kc, vc, n_pages, log2P, n_q, n_kv, M, max_ctx, out, st);
-}
 
 void launch_paged_attention(const AttnLaunch& a, hipStream_t st) {
   if (a.head_dim == 64)

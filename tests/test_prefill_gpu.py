@@ -355,6 +355,45 @@ def test_attention_prefill_max_ctx_caps_the_context(K):
         assert_close(out[m].view(n_q, D), ref, 2e-3, f"row {m}")
 
 
+@pytest.mark.parametrize("D,n_q,n_kv,page,start,M", [
+    (64, 8, 8, 16, 0, 31), (64, 8, 8, 16, 0, 33), (64, 32, 4, 16, 5, 127),      # edges of a wave's 32 columns
+    (64, 32, 4, 16, 0, 520), (64, 32, 4, 16, 100, 1550),                         # each workgroup shape, head dim 64
+    (128, 32, 8, 16, 0, 260), (128, 32, 8, 32, 63, 650), (128, 16, 8, 16, 0, 3080), (128, 32, 8, 16, 0, 4100),  # 128
+    (64, 8, 1, 1, 40, 70), (128, 8, 2, 2, 3, 90), (64, 32, 4, 4, 0, 1600), (128, 32, 8, 2, 0, 1550)])  # small pages
+def test_attention_prefill_workgroup_shapes(K, D, n_q, n_kv, page, start, M):
+    """Rows at the edges of tiles and blocks against the oracle in every workgroup shape of the launch rule (waves of
+    32 columns: up to 512 / 1536 / more at head dim 64, up to 256 / 640 / 1536 / 4095 / more at 128), and with pages
+    smaller than the rows of one load. 2e-3 as above: fp16 outputs of fp32 sums, p in about 22 bits."""
+    ctx_all = start + M
+    kc, vc, bt = make_cache(ctx_all, n_kv, page, D=D, seed=D + M + start)
+    qkv = torch.randn(M, (n_q + 2 * n_kv) * D, generator=gen(start + M)).half()
+    out = _prefill_attn(K, qkv, start, kc.to(DEV), vc.to(DEV), bt.to(DEV), n_q, n_kv, ctx_all).cpu()
+    for m in sorted({0, 1, 3, 4, 15, 16, 31, 32, 63, 64, 65, M // 2, M - 33, M - 2, M - 1} & set(range(M))):
+        q = qkv[m, : n_q * D].contiguous().view(n_q, D)
+        ref = R.paged_attention_ref(q, kc, vc, bt, start + m + 1, page)
+        assert_close(out[m].view(n_q, D), ref, 2e-3, f"row {m} vs oracle")
+
+
+@pytest.mark.parametrize("D,M", [(64, 40), (64, 1700), (128, 300), (128, 1700)])
+def test_attention_prefill_unmapped_page_reads_zeros(K, D, M):
+    """A block-table entry outside the cache gives zero K / V rows: the same bits as a page of zeros; an output that is
+    not 8-byte aligned is written all the same. Stale rows past the context (NaN here) reach nothing."""
+    n_q, n_kv, page = 16, 4, 16
+    kc, vc, bt = make_cache(M, n_kv, page, D=D, seed=3)
+    last = int(bt[(M - 1) // page])
+    kc[last, :, (M - 1) % page + 1:] = float("nan")
+    vc[last, :, (M - 1) % page + 1:] = float("nan")
+    qkv = torch.randn(M, (n_q + 2 * n_kv) * D, generator=gen(4)).half()
+    kz, vz, bt2 = kc.clone(), vc.clone(), bt.clone()
+    kz[int(bt[1])] = 0
+    vz[int(bt[1])] = 0
+    bt2[1] = -1
+    want = _prefill_attn(K, qkv, 0, kz.to(DEV), vz.to(DEV), bt.to(DEV), n_q, n_kv, M)
+    got = torch.empty(M * n_q * D + 1, dtype=torch.half, device=DEV)[1:].view(M, n_q * D)
+    K.attention_prefill(qkv.to(DEV), _pos(0), bt2.to(DEV), kc.to(DEV), vc.to(DEV), n_q, n_kv, M, got)
+    assert torch.isfinite(want).all() and torch.equal(got, want)
+
+
 # ---------------------------------------------------------------------------------------------------------------
 # Model.prefill
 
