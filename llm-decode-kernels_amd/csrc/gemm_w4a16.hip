@@ -7,7 +7,8 @@
 // fp16 integer and its fp16 product with the fp16 scale rounds the exact product once -- so every MFMA product is
 // exact and the sums are fp32. Epilogue 2 (split-K) writes fp32 partials instead of rows.
 //
-// Three kernels, chosen by grid size (gemm_w4a16_tile at the end of this file):
+// Up to 32 tokens take a kernel of their own (gemm_thin.hip). Three here, chosen by grid size (gemm_w4a16_tile at the
+// end of this file):
 //   * register-stationary (K % 128 == 0, G >= 64, a few hundred tiles of 256 weight rows): each wave's 64 weight
 //     rows are dequantized in registers straight into the v_mfma_f32_32x32x16_f16 A layout; only the token tile
 //     passes through LDS. The fastest form, described at its definition.
@@ -28,6 +29,7 @@
 //   W[col c][k 4g..4g+3]; the accumulator leaves lane l with Y[rows 4g..4g+3][col c].
 #include "common.hpp"
 #include "launch.hpp"
+#include "w4_common.hpp"
 
 namespace dk {
 namespace {
@@ -40,35 +42,6 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 __device__ __forceinline__ f4 mfma16(h4 a, h4 b, f4 c) { return __builtin_amdgcn_mfma_f32_16x16x16f16(a, b, c, 0, 0, 0); }
-
-// 8 weights of one packed word -> fp16((q - zero) * scale), in element order, given s2 = (scale, scale), zk = (1024 +
-// zero) twice and zs = (64 + zero) twice. Pairs (e0, e1) and (e4, e5) are nibbles 0 and 2 of each 16-bit half: OR-ed
-// into the mantissa of fp16 1024 (step 1) they give 1024 + q; pairs (e2, e3) and (e6, e7) are nibbles 1 and 3, and
-// OR-ed in place into fp16 64 (step 1/16) they give 64 + q, so one shift (by 8) serves all four pairs. Subtracting
-// 1024 + zero or 64 + zero is exact, and the product with the scale rounds the exact (q - zero) * scale once.
-// mlo = vgpr_const(0x000F000F), mhi = vgpr_const(0x00F000F0): one v_and_or_b32 per pair.
-__device__ __forceinline__ u32x4 dequant8_sz(uint32_t word, f16x2 s2, f16x2 zk, f16x2 zs, uint32_t mlo,
-                                             uint32_t mhi) {
-  const uint32_t hi = word >> 8;
-  const uint32_t p0 = (word & mlo) | 0x64006400u;
-  const uint32_t p1 = (word & mhi) | 0x54005400u;
-  const uint32_t p2 = (hi & mlo) | 0x64006400u;
-  const uint32_t p3 = (hi & mhi) | 0x54005400u;
-  u32x4 r;
-  r[0] = as_u32((as_f16x2(p0) - zk) * s2);
-  r[1] = as_u32((as_f16x2(p1) - zs) * s2);
-  r[2] = as_u32((as_f16x2(p2) - zk) * s2);
-  r[3] = as_u32((as_f16x2(p3) - zs) * s2);
-  return r;
-}
-
-// the same from the group's packed (scale, zero) pair (1024 + zero and 64 + zero are exact: zero is an integer in
-// [0, 15])
-__device__ __forceinline__ u32x4 dequant8(uint32_t word, uint32_t szw, uint32_t mlo, uint32_t mhi) {
-  const f16x2 sz = as_f16x2(szw);
-  const f16 zk = (f16)1024.0f + sz.y, zs = (f16)64.0f + sz.y;
-  return dequant8_sz(word, f16x2{sz.x, sz.x}, f16x2{zk, zk}, f16x2{zs, zs}, mlo, mhi);
-}
 
 template <int EPI>
 __global__ void __launch_bounds__(kGemmThreads)
@@ -425,7 +398,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint3
 
 // EPI 2 (split-K): the grid covers tiles x `splits` work items; item (tile, s) takes the k chunks [s nk / S,
 // (s + 1) nk / S) and writes its fp32 partial sums to Y = ws [S][M][N] (float), for gemm_splitk_reduce.
-template <int RW, int BM, int EPI>
+template <int RW, int BM, int EPI, bool FEW>
 __global__ void __launch_bounds__(kRsThreads, 2)
 gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M, int N, int K, int gsh,
               int tiles_m, int tiles, int splits) {
@@ -437,9 +410,9 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
   if (item >= tiles * splits) return;  // uniform: the grid is rounded up to a multiple of the XCD count
   // items are split-major with the token tiles fastest, so the tiles that share a weight tile's k range share an XCD
   const int t = item % tiles, split = item / tiles;
-  // a ragged last tile is shifted inward (the launcher requires M >= BM and N >= 256), so every row a lane loads is
+  // a ragged last tile is shifted inward (the launcher requires N >= 4 RW, and M >= BM unless FEW), so every row a lane loads is
   // valid; the rows it shares with its neighbour tile are computed by both, bit for bit alike, and stored twice
-  const int m0 = min((t % tiles_m) * BM, M - BM), n0 = min((t / tiles_m) * (4 * RW), N - 4 * RW);
+  const int m0 = FEW ? 0 : min((t % tiles_m) * BM, M - BM), n0 = min((t / tiles_m) * (4 * RW), N - 4 * RW);
   const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, h = lane >> 5;
   const int KW = K >> 3, NG = K >> gsh, nk_all = K / kRsK;
@@ -454,7 +427,11 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
   const uint32_t so = (row * (uint32_t)NG + (uint32_t)((64 * h) >> gsh)) * 4u;
   // X staging: chunk xq of rows xr + 16 v, stored at chunk xq ^ xr of the row (xr = (xr + 16 v) & 15)
   const int xq = tid & 15, xr = tid >> 4;
-  const uint32_t xo = (uint32_t)(m0 + xr) * (uint32_t)K * 2u + 16u * (uint32_t)xq;
+  // FEW (M < BM, one token tile): the rows past M are clamped, one offset each
+  uint32_t xo[FEW ? XL : 1];
+#pragma unroll
+  for (int v = 0; v < (FEW ? XL : 1); ++v)
+    xo[v] = (uint32_t)(FEW ? min(xr + 16 * v, M - 1) : m0 + xr) * (uint32_t)K * 2u + 16u * (uint32_t)xq;
 
   // with 128-token tiles X is staged in two halves of XL / 2 rows per thread, so only half a chunk of it is ever held
   // in registers (the accumulators leave no room for more); W and the scales are held for two chunks, the one
@@ -467,9 +444,13 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
   auto fetch_x = [&](int kc, int half) {
     const int k0 = (c_lo + min(kc, nk - 1)) * kRsK;
 #pragma unroll
-    for (int v = 0; v < XH; ++v)
-      xv[v] = __builtin_bit_cast(
-          u32x4, __builtin_amdgcn_raw_buffer_load_b128(xres, xo, 2 * k0 + 32 * K * (v + XH * half), 0));
+    for (int v = 0; v < XH; ++v) {
+      if constexpr (FEW)
+        xv[v] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xres, xo[v + XH * half], 2 * k0, 0));
+      else
+        xv[v] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xres, xo[0], 2 * k0 + 32 * K * (v + XH * half), 0));
+    }
   };
   auto fetch_w = [&](int kc, int slot) {
     const int k0 = (c_lo + min(kc, nk - 1)) * kRsK;
@@ -633,6 +614,7 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
           const int idx = lane + 64 * k2, t = idx / CPR, c = idx % CPR;
           const u32x4 v = *reinterpret_cast<const u32x4*>(reg + t * RB + ((c ^ (t & (CPR - 1))) << 4));
           const size_t m = (size_t)(m0 + 32 * j + t);
+          if (FEW && (int)m >= M) continue;
           if constexpr (EPI == 2)
             *reinterpret_cast<u32x4*>(reinterpret_cast<float*>(Y) + ((size_t)split * M + m) * N + nw0 + 4 * c) = v;
           else if constexpr (EPI == 1)
@@ -714,29 +696,41 @@ gemm_splitk_reduce(const float* __restrict__ ws, int splits, f16* __restrict__ Y
   reinterpret_cast<u32x2*>(Y)[i] = o;
 }
 
-// requires M >= BM and N >= 4 RW (the last tile in each direction is shifted inward); splits > 1: epilogue 0, N % 4
+void launch_splitk_reduce(const void* ws, int splits, void* y, int M, int N, hipStream_t st) {
+  const int mn4 = M * (N / 4);
+  hipLaunchKernelGGL(gemm_splitk_reduce, dim3((mn4 + 255) / 256), dim3(256), 0, st, (const float*)ws, splits, (f16*)y,
+                     mn4);
+}
+
+// requires M >= BM (or FEW) and N >= 4 RW (the last tile in each direction is shifted inward); splits > 1: epilogue 0, N % 4
 // == 0 and a workspace of splits * M * N floats (the partials), reduced by a second launch
-template <int RW, int BM>
-void launch_rs(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
-               int epilogue, int splits, void* ws, hipStream_t st) {
+template <int RW, int BM, bool FEW>
+void launch_rs_m(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
+                 int epilogue, int splits, void* ws, hipStream_t st) {
   const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + 4 * RW - 1) / (4 * RW));
   const dim3 grid((tiles * splits + kXcds - 1) / kXcds * kXcds);
   const uint32_t* P = (const uint32_t*)packed;
   const uint32_t* S = (const uint32_t*)sz;
   if (splits > 1) {
-    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 2>), grid, dim3(kRsThreads), 0, st, P, S, (const f16*)x, (f16*)ws, M, N,
-                       K, log2G, tiles_m, tiles, splits);
-    if (epilogue == 2) return;  // the partials are the output (their reader sums them)
-    const int mn4 = M * (N / 4);
-    hipLaunchKernelGGL(gemm_splitk_reduce, dim3((mn4 + 255) / 256), dim3(256), 0, st, (const float*)ws, splits,
-                       (f16*)y, mn4);
+    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 2, FEW>), grid, dim3(kRsThreads), 0, st, P, S, (const f16*)x, (f16*)ws, M,
+                       N, K, log2G, tiles_m, tiles, splits);
+    if (epilogue != 2) launch_splitk_reduce(ws, splits, y, M, N, st);  // 2: the reader of the partials sums them
   } else if (epilogue == 1) {
-    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 1>), grid, dim3(kRsThreads), 0, st, P, S, (const f16*)x, (f16*)y, M, N, K,
-                       log2G, tiles_m, tiles, 1);
+    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 1, FEW>), grid, dim3(kRsThreads), 0, st, P, S, (const f16*)x, (f16*)y, M,
+                       N, K, log2G, tiles_m, tiles, 1);
   } else {
-    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 0>), grid, dim3(kRsThreads), 0, st, P, S, (const f16*)x, (f16*)y, M, N, K,
-                       log2G, tiles_m, tiles, 1);
+    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 0, FEW>), grid, dim3(kRsThreads), 0, st, P, S, (const f16*)x, (f16*)y, M,
+                       N, K, log2G, tiles_m, tiles, 1);
   }
+}
+template <int RW, int BM>
+void launch_rs(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
+               int epilogue, int splits, void* ws, hipStream_t st) {
+  if constexpr (RW == 32 && BM == 64) {
+    if (M < BM)
+      return launch_rs_m<RW, BM, true>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
+  }
+  launch_rs_m<RW, BM, false>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
 }
 
 #ifndef DK_GEMM_PD
@@ -776,7 +770,7 @@ void launch_wide(const void* packed, const void* sz, const void* x, void* y, int
 #ifndef DK_GEMM_RS
 #define DK_GEMM_RS 1
 #endif
-// Split-K (a workspace given, epilogue 0 or 2 = the partials alone, K % 128 == 0, G >= 64, M >= 64, N >= 256, N % 4 == 0, offsets within 31
+// Split-K (a workspace given, epilogue 0 or 2 = the partials alone, K % 128 == 0, G >= 64, M >= 33, N >= 256, N % 4 == 0, offsets within 31
 // bits): taken when no unsplit register-stationary tiling has its tiles (gemm_w4a16_rs_tile) or K is long (64 chunks
 // of 128 or more: Llama-3-8B down 4096 x 14336 at M 512 takes 82 us split 4 ways against 92 unsplit on 128-row
 // tiles, while its o 4096 x 4096 takes 28.5 unsplit against 31.6 split). Over 64-token tiles of 256 weight rows, else
@@ -784,23 +778,42 @@ void launch_wide(const void* packed, const void* sz, const void* x, void* y, int
 // least 16 of the 128-wide chunks, and only if S x tiles reaches 192. Shorter splits lose: the partials' traffic
 // (S x M x N x 4 bytes, written and read back) and the reduce launch outweigh the fuller grid (TinyLlama qkv
 // 2560 x 2048 at S 4, 4 chunks per split: 27 against 19 us). Returns S (1: no split) and the rows per wave in *rw.
-constexpr int kSplitMinChunks = 16;
+// Up to 128 tokens the partials are small and the alternative is the wide kernel with a few tiles, so there shorter
+// splits (5 chunks) over 128-row tiles pay while the tiles alone leave three quarters of the CUs idle: 4096 x 14336 at M 64
+// 20.8 us against 66.2, 4096 x 4096 at M 33 / 64 / 128 13.0 / 13.6 / 16.3 against 18.9 / 20.5 / 19.9, 2048 x 5632 at 64
+// 12.0 against 26.4; with 96 tiles (6144 x 4096 at M 128) they lose, 21 against 19.2.
+// Fewer than 64 tokens (FEW) run on the 64-token tile down to 33 (28672 x 4096 at M 48: 29.7 us against 46.4 on the wide
+// kernel); up to 32 take the thin kernel (gemm_thin.hip).
+constexpr int kSplitMinChunks = 16, kRsMinM = 33;
 int gemm_w4a16_rs_tile(int M, int N, int K, int log2G);
 
 int gemm_w4a16_splits(int M, int N, int K, int log2G, int epilogue, int* rw) {
   *rw = 64;
-  if (!DK_GEMM_RS || (epilogue != 0 && epilogue != 2) || K % kRsK != 0 || log2G < 6 || M < 64 || N < 256 || N % 4 != 0 ||
+  if ((epilogue == 0 || epilogue == 2) && gemm_thin_fits(M, N, K, log2G)) {
+    *rw = 0;
+    return gemm_thin_splits(M, N, K, log2G);
+  }
+  if (!DK_GEMM_RS || (epilogue != 0 && epilogue != 2) || K % kRsK != 0 || log2G < 6 || M < kRsMinM || N < 256 || N % 4 != 0 ||
       (long long)N * K > 0x7fffffffLL || (long long)M * K > 0x3fffffffLL)
     return 1;
   const int nk = K / kRsK;
   if (nk < 64 && gemm_w4a16_rs_tile(M, N, K, log2G) != 0) return 1;
   const long long tm = (M + 63) / 64;
-  for (int r = 64; r >= 32; r /= 2) {
+  for (int r = M < 64 ? 32 : 64; r >= 32; r /= 2) {
     const long long tiles = (N + 4 * r - 1) / (4 * r) * tm;
     int s = 2;
     while (s < 16 && tiles * s < 384 && nk / (2 * s) >= kSplitMinChunks) s *= 2;
     if (nk / s >= kSplitMinChunks && tiles * s >= 192) {
       *rw = r;
+      return s;
+    }
+  }
+  if (M <= 128) {
+    const long long tiles = (N + 127) / 128 * tm;
+    int s = 2;
+    while (s < 16 && tiles * s < 192 && nk / (2 * s) >= 5) s *= 2;
+    if (tiles <= 64 && nk / s >= 5 && tiles * s >= 128) {
+      *rw = 32;
       return s;
     }
   }
@@ -821,7 +834,7 @@ int gemm_w4a16_rs_tile(int M, int N, int K, int log2G) {
   const long long n_t = (N + 255) / 256, n_t32 = (N + 127) / 128, tm128 = (M + 127) / 128, tm64 = (M + 63) / 64;
   if (M >= 128 && N >= 256 && n_t * tm128 >= 320) return 42;
   if (M >= 128 && N >= 128 && n_t32 * tm128 >= 320) return 52;
-  if (M >= 64 && N >= 128 && n_t32 * tm64 >= 160) return 51;
+  if (M >= kRsMinM && N >= 128 && n_t32 * tm64 >= 160) return 51;
   return 0;
 }
 
@@ -854,10 +867,16 @@ void launch_gemm_w4a16(const void* packed, const void* sz, const void* x, void* 
     int rw;
     const int splits = gemm_w4a16_splits(M, N, K, log2G, epilogue, &rw);
     if (splits > 1) {
+      if (rw == 0) {
+        launch_gemm_thin(packed, sz, x, ws, M, N, K, log2G, 2, splits, st);
+        if (epilogue != 2) launch_splitk_reduce(ws, splits, y, M, N, st);
+        return;
+      }
       if (rw == 64) return launch_rs<64, 64>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
       return launch_rs<32, 64>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
     }
   }
+  if (gemm_thin_fits(M, N, K, log2G)) return launch_gemm_thin(packed, sz, x, y, M, N, K, log2G, epilogue, 1, st);
   switch (gemm_w4a16_tile(M, N, K, log2G)) {
     case 42: launch_rs<64, 128>(packed, sz, x, y, M, N, K, log2G, epilogue, 1, nullptr, st); return;
     case 52: launch_rs<32, 128>(packed, sz, x, y, M, N, K, log2G, epilogue, 1, nullptr, st); return;

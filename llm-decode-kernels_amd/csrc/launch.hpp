@@ -77,6 +77,13 @@ void launch_gemm_w4a16(const void* packed, const void* sz, const void* x, void* 
 // bytes of fp32 split-K partials launch_gemm_w4a16 uses for this shape when given a workspace (0: it does not split)
 size_t gemm_w4a16_workspace_bytes(int M, int N, int K, int log2G, int epilogue);
 
+// The GEMM of a few tokens (gemm_thin.hip): whether a shape takes it, the k ranges it splits into when a workspace is
+// given (1: it does not split), and its launch (splits > 1: y receives the fp32 partials [splits, M, N]).
+bool gemm_thin_fits(int M, int N, int K, int log2G);
+int gemm_thin_splits(int M, int N, int K, int log2G);
+void launch_gemm_thin(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
+                      int epilogue, int splits, hipStream_t st);
+
 // Read-ceiling probe (read_probe.hip): `blocks` workgroups of `threads` threads, workgroup b streaming the b-th of
 // `blocks` equal contiguous slabs in rounds of depth x threads 16-byte words; with sink_words >= blocks x W (W =
 // threads / 64) sink[b W + w] receives the sum of the 32-bit words wave w of workgroup b read, else nothing is written.

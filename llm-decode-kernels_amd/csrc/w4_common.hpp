@@ -54,4 +54,33 @@ __device__ __forceinline__ float column_row(const u32x4& w, float z, const u32x4
   return fmaf(-z, cs.S, d);
 }
 
+// 8 weights of one packed word -> fp16((q - zero) * scale), in element order, given s2 = (scale, scale), zk = (1024 +
+// zero) twice and zs = (64 + zero) twice. Pairs (e0, e1) and (e4, e5) are nibbles 0 and 2 of each 16-bit half: OR-ed
+// into the mantissa of fp16 1024 (step 1) they give 1024 + q; pairs (e2, e3) and (e6, e7) are nibbles 1 and 3, and
+// OR-ed in place into fp16 64 (step 1/16) they give 64 + q, so one shift (by 8) serves all four pairs. Subtracting
+// 1024 + zero or 64 + zero is exact, and the product with the scale rounds the exact (q - zero) * scale once.
+// mlo = vgpr_const(0x000F000F), mhi = vgpr_const(0x00F000F0): one v_and_or_b32 per pair.
+__device__ __forceinline__ u32x4 dequant8_sz(uint32_t word, f16x2 s2, f16x2 zk, f16x2 zs, uint32_t mlo,
+                                             uint32_t mhi) {
+  const uint32_t hi = word >> 8;
+  const uint32_t p0 = (word & mlo) | 0x64006400u;
+  const uint32_t p1 = (word & mhi) | 0x54005400u;
+  const uint32_t p2 = (hi & mlo) | 0x64006400u;
+  const uint32_t p3 = (hi & mhi) | 0x54005400u;
+  u32x4 r;
+  r[0] = as_u32((as_f16x2(p0) - zk) * s2);
+  r[1] = as_u32((as_f16x2(p1) - zs) * s2);
+  r[2] = as_u32((as_f16x2(p2) - zk) * s2);
+  r[3] = as_u32((as_f16x2(p3) - zs) * s2);
+  return r;
+}
+
+// the same from the group's packed (scale, zero) pair (1024 + zero and 64 + zero are exact: zero is an integer in
+// [0, 15])
+__device__ __forceinline__ u32x4 dequant8(uint32_t word, uint32_t szw, uint32_t mlo, uint32_t mhi) {
+  const f16x2 sz = as_f16x2(szw);
+  const f16 zk = (f16)1024.0f + sz.y, zs = (f16)64.0f + sz.y;
+  return dequant8_sz(word, f16x2{sz.x, sz.x}, f16x2{zk, zk}, f16x2{zs, zs}, mlo, mhi);
+}
+
 }  // namespace dk

@@ -179,6 +179,35 @@ def test_gemm_splitk_one_hot_rows_exact(K):
     assert torch.equal(y.cpu(), wref[:, ks].t().contiguous())
 
 
+# few tokens: the thin kernel at 128, 64, 32 and 16 weight rows per workgroup (ragged N, K not a multiple of 256, more
+# chunks than groups by a remainder, so that some groups end on a chunk of zeros) and its split-K; the 64-token
+# register-stationary tile with fewer tokens, unsplit and split, and short splits up to 128 tokens
+@pytest.mark.parametrize("M,N,Kd,G,S", [(1, 20484, 1024, 64, 0), (16, 20501, 1152, 64, 0), (17, 10250, 1280, 128, 0),
+                                        (32, 5130, 1152, 128, 0), (31, 2049, 1408, 64, 0), (2, 1900, 2176, 64, 0),
+                                        (15, 4100, 8192, 256, 4), (32, 4096, 14336, 128, 8), (33, 20500, 256, 64, 0),
+                                        (63, 20493, 384, 64, 0), (47, 4100, 5120, 64, 8), (128, 2052, 5632, 128, 8),
+                                        (65, 4096, 4096, 128, 4)])
+def test_gemm_few_tokens_exact_on_integer_grid(K, M, N, Kd, G, S):
+    """As test_gemm_exact_on_integer_grid: bit-exact, with and without the workspace; the SwiGLU epilogue
+    against the oracle's swiglu of the exact rows (1e-3: its silu is fp32 as here, rounded to fp16 twice)."""
+    packed, sz, wref = _grid_weights(N, Kd, G, seed=M + N + Kd)
+    x = torch.randint(-3, 4, (M, Kd), generator=gen(M + 1)).half()
+    want = (x.double() @ wref.double().t()).half()      # exact sums, one rounding
+    need = K.gemm_workspace_bytes(M, N, Kd, G)
+    assert need == S * M * N * 4
+    for ws in (None, torch.full((need,), 0xFF, dtype=torch.uint8, device=DEV) if need else None):
+        y = torch.full((M, N), 7.0, dtype=torch.half, device=DEV)
+        K.gemm_w4a16(packed, sz, x.to(DEV), y, G, workspace=ws)
+        assert torch.equal(y.cpu(), want)
+    if need:
+        parts = K.gemm_w4a16_parts(packed, sz, x.to(DEV), G, torch.empty(need, dtype=torch.uint8, device=DEV))
+        assert torch.equal(parts.double().sum(0).half().cpu(), want)
+    if N % 2 == 0:
+        act = torch.full((M, N // 2), 7.0, dtype=torch.half, device=DEV)
+        K.gemm_w4a16(packed, sz, x.to(DEV), act, G, epilogue=1)
+        assert_close(act, R.swiglu_ref(torch.cat([want[:, 0::2], want[:, 1::2]], 1)), 1e-3, "swiglu of the exact rows")
+
+
 @pytest.mark.parametrize("N", [200, 49152])
 def test_gemm_one_hot_rows_exact(K, N):
     """Row i of X is one-hot at k_i, so row i of Y is column k_i of the dequantized weight, bit for bit (N 49152 runs
