@@ -7,9 +7,8 @@
 // fp16 integer and its fp16 product with the fp16 scale rounds the exact product once -- so every MFMA product is
 // exact and the sums are fp32. Epilogue 2 (split-K) writes fp32 partials instead of rows.
 //
-// Up to 32 tokens take a kernel of their own (gemm_thin.hip). Three here, chosen by grid size (gemm_w4a16_tile at the
-// end of this file):
-//   * register-stationary (K % 128 == 0, G >= 64, a few hundred tiles of 256 weight rows): each wave's 64 weight
+// Up to 32 tokens take a kernel of their own (gemm_thin.hip). Three here, chosen by grid size (the end of this file):
+//   * register-stationary (K % 128 == 0, G >= 64, M >= 33, a grid that fills the CUs): each wave's 64 or 32 weight
 //     rows are dequantized in registers straight into the v_mfma_f32_32x32x16_f16 A layout; only the token tile
 //     passes through LDS. The fastest form, described at its definition.
 //   * wide (K % 64 == 0): weight and token tiles of 64 or 128 both staged in LDS (the weights dequantized on the
@@ -370,20 +369,14 @@ gemm_w4a16_wide(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int
 //   and their sums are those of the plain order. The accumulator of tile (i, j) leaves lane (h, r) with rows
 //   8 q + 4 h + v (q, v = 0..3) of the weight tile for token r: four consecutive outputs of one token per q.
 //   LDS traffic: per k step a wave reads BM / 32 token fragments of 1 KB for 2 BM / 32 MFMAs of 32 cycles, 8 bytes
-//   per MFMA cycle, 32 per CU cycle with four waves at the full MFMA rate, plus the stage's 16.
+//   per MFMA cycle, 32 per CU cycle with four waves at the full MFMA rate, plus the stage's 16 (8 with eight waves).
 // Pipeline per chunk c: compute chunk c (dequant of W(c) in registers, one k step ahead of the MFMAs; X(c) from LDS
 // buffer c & 1); halfway through, store the first half of X(c + 1) (loaded a chunk earlier) into the other buffer and
 // load its second half; after the MFMAs store that half, issue the loads of X(c + 2)'s first half and W(c + 2), barrier. W, scales and X come in
 // through buffer loads (SGPR base and chunk offset, a constant VGPR offset per row), so moving to the next chunk costs
-// no vector instruction; the host checks that every offset fits 31 bits. Two workgroups share a CU (accumulators and
-// operands in the 256 architectural VGPRs of a wave).
-constexpr int kRsK = 128, kRsThreads = 256;
-#ifndef RS_AHEAD
-#define RS_AHEAD 3
-#endif
-#ifndef RS_XSPLIT
-#define RS_XSPLIT (KS * TJ / 2)
-#endif
+// no vector instruction; the host checks that every offset fits 31 bits. Two waves share a SIMD (accumulators and
+// operands in the 256 architectural VGPRs of a wave): two workgroups of four waves, or one of eight.
+constexpr int kRsK = 128;
 
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
@@ -398,12 +391,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint3
 
 // EPI 2 (split-K): the grid covers tiles x `splits` work items; item (tile, s) takes the k chunks [s nk / S,
 // (s + 1) nk / S) and writes its fp32 partial sums to Y = ws [S][M][N] (float), for gemm_splitk_reduce.
-template <int RW, int BM, int EPI, bool FEW>
-__global__ void __launch_bounds__(kRsThreads, 2)
+template <int RW, int BM, int EPI, int NW, bool FEW>
+__global__ void __launch_bounds__(NW * kWave, 2)
 gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M, int N, int K, int gsh,
               int tiles_m, int tiles, int splits) {
   constexpr int TI = RW / 32, TJ = BM / 32, KS = kRsK / 16;
-  constexpr int XL = BM * 16 / kRsThreads;  // 16-byte X loads per thread per chunk
+  constexpr int XR = NW * kWave / 16;       // token rows per X load index
+  constexpr int XL = BM / XR;               // 16-byte X loads per thread per chunk
   __shared__ u32x4 Xs[2][BM][16];
   const int per = gridDim.x / kXcds;
   const int item = (int)(blockIdx.x % kXcds) * per + (int)(blockIdx.x / kXcds);
@@ -412,7 +406,7 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
   const int t = item % tiles, split = item / tiles;
   // a ragged last tile is shifted inward (the launcher requires N >= 4 RW, and M >= BM unless FEW), so every row a lane loads is
   // valid; the rows it shares with its neighbour tile are computed by both, bit for bit alike, and stored twice
-  const int m0 = FEW ? 0 : min((t % tiles_m) * BM, M - BM), n0 = min((t / tiles_m) * (4 * RW), N - 4 * RW);
+  const int m0 = FEW ? 0 : min((t % tiles_m) * BM, M - BM), n0 = min((t / tiles_m) * (NW * RW), N - NW * RW);
   const int tid = (int)threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, h = lane >> 5;
   const int KW = K >> 3, NG = K >> gsh, nk_all = K / kRsK;
@@ -425,18 +419,18 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
   const uint32_t row = (uint32_t)(n0 + wave * RW + r);
   const uint32_t wo = row * (uint32_t)KW * 4u + 32u * (uint32_t)h;
   const uint32_t so = (row * (uint32_t)NG + (uint32_t)((64 * h) >> gsh)) * 4u;
-  // X staging: chunk xq of rows xr + 16 v, stored at chunk xq ^ xr of the row (xr = (xr + 16 v) & 15)
+  // X staging: chunk xq of rows xr + XR v (XR a multiple of 16), stored at chunk xq ^ (xr & 15) of the row
   const int xq = tid & 15, xr = tid >> 4;
   // FEW (M < BM, one token tile): the rows past M are clamped, one offset each
   uint32_t xo[FEW ? XL : 1];
 #pragma unroll
   for (int v = 0; v < (FEW ? XL : 1); ++v)
-    xo[v] = (uint32_t)(FEW ? min(xr + 16 * v, M - 1) : m0 + xr) * (uint32_t)K * 2u + 16u * (uint32_t)xq;
+    xo[v] = (uint32_t)(FEW ? min(xr + XR * v, M - 1) : m0 + xr) * (uint32_t)K * 2u + 16u * (uint32_t)xq;
 
   // with 128-token tiles X is staged in two halves of XL / 2 rows per thread, so only half a chunk of it is ever held
   // in registers (the accumulators leave no room for more); W and the scales are held for two chunks, the one
   // computed and the next
-  constexpr int NXH = BM >= 128 ? 2 : 1, XH = XL / NXH;
+  constexpr int NXH = XL > 4 ? 2 : 1, XH = XL / NXH;
   u32x4 xv[XH], wv[2][TI][2];
   uint32_t sv[2][TI];
   // loads are unconditional (chunks past the end re-read the last one): a load behind a branch would make the
@@ -449,7 +443,7 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
         xv[v] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xres, xo[v + XH * half], 2 * k0, 0));
       else
         xv[v] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xres, xo[0], 2 * k0 + 32 * K * (v + XH * half), 0));
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xres, xo[0], 2 * k0 + 2 * XR * K * (v + XH * half), 0));
     }
   };
   auto fetch_w = [&](int kc, int slot) {
@@ -467,7 +461,7 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
   };
   auto stage = [&](int buf, int half) {
 #pragma unroll
-    for (int v = 0; v < XH; ++v) Xs[buf][xr + 16 * (v + XH * half)][xq ^ xr] = xv[v];
+    for (int v = 0; v < XH; ++v) Xs[buf][xr + XR * (v + XH * half)][xq ^ (xr & 15)] = xv[v];
   };
   f32x16 acc[TI][TJ];
 #pragma unroll
@@ -477,7 +471,7 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
   }
   const uint32_t mlo = vgpr_const(0x000F000Fu), mhi = vgpr_const(0x00F000F0u);
   // MFMAs of one chunk; `mid` (the next chunk's first X half into LDS, its second half's loads) runs after the
-  // MFMAs of the first RS_XSPLIT fragments
+  // MFMAs of the chunk's first half
   auto compute = [&](int buf, int slot, auto&& mid) {
     // the chunk's weight words and scales enter here: without the pin the compiler hoists their first use above the
     // previous chunk's barrier, where waiting for them drains the newer loads as well
@@ -497,7 +491,7 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
     }
     // the chunk's KS x TJ token fragments in (k step, token tile) order, each read from LDS RB fragments ahead of
     // its MFMAs so the reads' latency hides behind the MFMAs of the ones before it
-    constexpr int NB = KS * TJ, RB = RS_AHEAD;
+    constexpr int NB = KS * TJ, RB = 3;
     h8 b[RB + 1];
     auto read_b = [&](int q) {
       return __builtin_bit_cast(h8, Xs[buf][32 * (q % TJ) + r][(8 * h + q / TJ) ^ (r & 15)]);
@@ -515,7 +509,7 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
 #pragma unroll
     for (int q = 0; q < NB; ++q) {
       const int s = q / TJ;
-      if (q == RS_XSPLIT) mid();
+      if (q == NB / 2) mid();
       if (q + RB < NB) b[(q + RB) % (RB + 1)] = read_b(q + RB);
 #pragma unroll
       for (int i = 0; i < TI; ++i) acc[i][q % TJ] = mfma32x32(a[s & 1][i], b[q % (RB + 1)], acc[i][q % TJ]);
@@ -574,7 +568,7 @@ gemm_w4a16_rs(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int M
   {
     constexpr int ES = EPI == 2 ? 4 : (EPI == 1 ? 1 : 2);  // output bytes per weight row and token
     constexpr int RB = RW * ES, CPR = RB / 16;              // a token's bytes in the wave's slice, its 16-byte chunks
-    static_assert(CPR >= 2 && 32 * CPR % 64 == 0 && 4 * 32 * RB <= (int)sizeof(Xs), "staged epilogue fits");
+    static_assert(CPR >= 2 && 32 * CPR % 64 == 0 && NW * 32 * RB <= (int)sizeof(Xs), "staged epilogue fits");
     const bool co = (reinterpret_cast<uintptr_t>(Y) & 15) == 0 &&  // 16-byte aligned rows (uniform)
                     (EPI == 2 || (EPI == 0 ? (N & 7) == 0 : (N & 15) == 0));
     if (co) {
@@ -704,40 +698,27 @@ void launch_splitk_reduce(const void* ws, int splits, void* y, int M, int N, hip
 
 // requires M >= BM (or FEW) and N >= 4 RW (the last tile in each direction is shifted inward); splits > 1: epilogue 0, N % 4
 // == 0 and a workspace of splits * M * N floats (the partials), reduced by a second launch
-template <int RW, int BM, bool FEW>
-void launch_rs_m(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
-                 int epilogue, int splits, void* ws, hipStream_t st) {
-  const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + 4 * RW - 1) / (4 * RW));
-  const dim3 grid((tiles * splits + kXcds - 1) / kXcds * kXcds);
+template <int RW, int BM, int NW = 4, bool FEW = false>
+void launch_rs(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
+               int epilogue, int splits, void* ws, hipStream_t st) {
+  const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + NW * RW - 1) / (NW * RW));
+  const dim3 grid((tiles * splits + kXcds - 1) / kXcds * kXcds), block(NW * kWave);
   const uint32_t* P = (const uint32_t*)packed;
   const uint32_t* S = (const uint32_t*)sz;
   if (splits > 1) {
-    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 2, FEW>), grid, dim3(kRsThreads), 0, st, P, S, (const f16*)x, (f16*)ws, M,
-                       N, K, log2G, tiles_m, tiles, splits);
+    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 2, NW, FEW>), grid, block, 0, st, P, S, (const f16*)x, (f16*)ws, M, N, K,
+                       log2G, tiles_m, tiles, splits);
     if (epilogue != 2) launch_splitk_reduce(ws, splits, y, M, N, st);  // 2: the reader of the partials sums them
   } else if (epilogue == 1) {
-    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 1, FEW>), grid, dim3(kRsThreads), 0, st, P, S, (const f16*)x, (f16*)y, M,
-                       N, K, log2G, tiles_m, tiles, 1);
+    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 1, NW, FEW>), grid, block, 0, st, P, S, (const f16*)x, (f16*)y, M, N, K,
+                       log2G, tiles_m, tiles, 1);
   } else {
-    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 0, FEW>), grid, dim3(kRsThreads), 0, st, P, S, (const f16*)x, (f16*)y, M,
-                       N, K, log2G, tiles_m, tiles, 1);
+    hipLaunchKernelGGL((gemm_w4a16_rs<RW, BM, 0, NW, FEW>), grid, block, 0, st, P, S, (const f16*)x, (f16*)y, M, N, K,
+                       log2G, tiles_m, tiles, 1);
   }
 }
-template <int RW, int BM>
-void launch_rs(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
-               int epilogue, int splits, void* ws, hipStream_t st) {
-  if constexpr (RW == 32 && BM == 64) {
-    if (M < BM)
-      return launch_rs_m<RW, BM, true>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
-  }
-  launch_rs_m<RW, BM, false>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
-}
 
-#ifndef DK_GEMM_PD
-#define DK_GEMM_PD 2
-#endif
-
-template <int BN, int BM, int KG, int PD = DK_GEMM_PD>
+template <int BN, int BM, int KG, int PD = 2>
 void launch_wide(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
                  int epilogue, hipStream_t st) {
   const int tiles_m = (M + BM - 1) / BM, tiles = tiles_m * ((N + BN - 1) / BN);
@@ -752,96 +733,148 @@ void launch_wide(const void* packed, const void* sz, const void* x, void* y, int
                        tiles);
 }
 
-}  // namespace
 
-// Tile choice: the register-stationary kernel (K % 128 == 0, G >= 64) in the first of these that gives its number
-// of tiles (two workgroups per CU: 512 slots): 256 weight rows x 128 tokens, 320 tiles (returns 42); 128 x 128, 320
-// (52); 128 x 64, 160 (51). The 128-row tiles (32 rows per wave) give the narrower shapes their tiles (TinyLlama qkv
-// 2560 x 2048 at M 512: 14.0 against 17.3 us on the wide kernel; gate|up 11264 x 2048: 37.1 against 40.3 at 256 x 64;
-// Llama-3-8B qkv 6144 x 4096: 40.0 against 41.4 at 256 x 64, 384 tiles against 192, which is why 256 x 64 tiles are
-// no longer among the unsplit choices: wherever they reach 160 tiles the 128 x 64 tiling reaches 320); below 160
-// they lose to the wide kernel (TinyLlama o and down: 13.8 against 11.4 and 34.2 against 31.3 us at 128 tiles). Otherwise the wide kernel: the largest of 128 x 128, 128 x 64, 64 x 64 whose grid still covers the 256
-// CUs, then K groups (KG = 2 or 4 four-wave groups per workgroup; 2 at most for 128 x 64, by LDS) while the grid leaves
-// CUs with a single workgroup (returns 10 * tile + KG, tile 3: 128 x 128, 2: 128 x 64, 1: 64 x 64); K % 64 != 0 takes
-// the 64 x 64 16x16x16 kernel above (returns 0).
-#ifndef DK_GEMM_KG
-#define DK_GEMM_KG 0
-#endif
-#ifndef DK_GEMM_RS
-#define DK_GEMM_RS 1
-#endif
-// Split-K (a workspace given, epilogue 0 or 2 = the partials alone, K % 128 == 0, G >= 64, M >= 33, N >= 256, N % 4 == 0, offsets within 31
-// bits): taken when no unsplit register-stationary tiling has its tiles (gemm_w4a16_rs_tile) or K is long (64 chunks
-// of 128 or more: Llama-3-8B down 4096 x 14336 at M 512 takes 82 us split 4 ways against 92 unsplit on 128-row
-// tiles, while its o 4096 x 4096 takes 28.5 unsplit against 31.6 split). Over 64-token tiles of 256 weight rows, else
-// 128: the smallest power-of-two split S in 2..16 whose S x tiles reaches 384 workgroups while every split keeps at
-// least 16 of the 128-wide chunks, and only if S x tiles reaches 192. Shorter splits lose: the partials' traffic
-// (S x M x N x 4 bytes, written and read back) and the reduce launch outweigh the fuller grid (TinyLlama qkv
-// 2560 x 2048 at S 4, 4 chunks per split: 27 against 19 us). Returns S (1: no split) and the rows per wave in *rw.
-// Up to 128 tokens the partials are small and the alternative is the wide kernel with a few tiles, so there shorter
-// splits (5 chunks) over 128-row tiles pay while the tiles alone leave three quarters of the CUs idle: 4096 x 14336 at M 64
-// 20.8 us against 66.2, 4096 x 4096 at M 33 / 64 / 128 13.0 / 13.6 / 16.3 against 18.9 / 20.5 / 19.9, 2048 x 5632 at 64
-// 12.0 against 26.4; with 96 tiles (6144 x 4096 at M 128) they lose, 21 against 19.2.
-// Fewer than 64 tokens (FEW) run on the 64-token tile down to 33 (28672 x 4096 at M 48: 29.7 us against 46.4 on the wide
-// kernel); up to 32 take the thin kernel (gemm_thin.hip).
-constexpr int kSplitMinChunks = 16, kRsMinM = 33;
-int gemm_w4a16_rs_tile(int M, int N, int K, int log2G);
+// Tilings of the register-stationary kernel: weight rows per wave, tokens, waves per workgroup (rows x waves = the
+// tile's weight rows), and the output a CU makes in a given time when it has a full tile, relative to the first (chunk
+// time of a CU-filling grid: 512 x 128 3.5 us, 256 x 128 2.0, 256 x 64 1.2; two 256 x 128 tiles of four waves 3.9, one
+// 2.1). Eight-wave tiles share each staged X among twice the rows (with the staging taken out of the four-wave kernel,
+// 28672 x 4096 at M 512 runs in 114 us instead of 132), four-wave ones drain more smoothly over many rounds.
+enum RsId { kRsNone, kRs512x128, kRs256x128, kRs256x64, kRs256x128w4, kRs128x128w4, kRs128x64w4 };
+struct RsTiling {
+  RsId id;
+  int rw, bm, nw;
+  double rate;
+};
+constexpr RsTiling kRsTilings[] = {
+    {kRs512x128, 64, 128, 8, 1.0},    {kRs256x128, 32, 128, 8, 0.875},  {kRs256x64, 32, 64, 8, 0.73},
+    {kRs256x128w4, 64, 128, 4, 0.88}, {kRs128x128w4, 32, 128, 4, 0.72}, {kRs128x64w4, 32, 64, 4, 0.64}};
+constexpr int kCus = 256, kRsMinM = 33;
 
-int gemm_w4a16_splits(int M, int N, int K, int log2G, int epilogue, int* rw) {
-  *rw = 64;
-  if ((epilogue == 0 || epilogue == 2) && gemm_thin_fits(M, N, K, log2G)) {
-    *rw = 0;
-    return gemm_thin_splits(M, N, K, log2G);
+// The tiling with the most output per time over S k ranges of an M x N output: its rate times the share of the CUs'
+// tile area that is output, rounds of 256 tiles counted whole. Measured against the tiling that the count of tiles
+// alone chose before, us: 28672 x 4096 at M 333 / 512 / 1024 101 / 117.6 / 231.6 (512 x 128) against 117 / 124 / 247
+// (256 x 128, four waves; at M 2048 that one keeps, 456 against 464); 11264 x 2048 at 333 / 512 29.8 / 32.1 (256 x 128)
+// against 34.8 / 35.7, at 1024 56.7 (512 x 128) against 62.1; 6144 x 4096 at 512 / 1024 / 2048 38.1 / 58.2 / 104.7
+// against 42.7 / 65.0 / 115; 4096 x 4096 at 2048 70.0 against 74.8; 2560 x 2048 at 1024 / 2048 20.0 / 30.5 against
+// 22.5 / 33.1; 2048 x 2048 at 2048 24.2 against 27.1.
+RsTiling rs_best(int M, int N, int S, double* score) {
+  RsTiling best = {kRsNone, 0, 0, 0, 0.0};
+  *score = 0.0;
+  for (const RsTiling& t : kRsTilings) {
+    if (N < t.nw * t.rw || (M < t.bm && !(t.id == kRs128x64w4 && M >= kRsMinM))) continue;
+    const long long tiles = (long long)((N + t.nw * t.rw - 1) / (t.nw * t.rw)) * ((M + t.bm - 1) / t.bm) * S;
+    double rounds = (double)((tiles + kCus - 1) / kCus), rate = t.rate;
+    if (t.nw == 4 && t.bm == 128 && tiles > 2 * kCus) {
+      // CUs refill one workgroup at a time (6144 x 4096 at M 1500: 128 x 128 tiles in 2.25 rounds 99 us, 512 x 128 ones
+      // in 0.56 of a round 109)
+      rounds = (double)tiles / kCus + 0.3;
+      rate *= 1.045;
+    } else if (t.id == kRs256x128w4 && tiles <= kCus) {
+      rate = 0.81;  // one workgroup per CU
+    }
+    const double sc = rate * M * N * S / (rounds * kCus * t.nw * t.rw * t.bm);
+    if (sc > *score) {
+      *score = sc;
+      best = t;
+    }
   }
-  if (!DK_GEMM_RS || (epilogue != 0 && epilogue != 2) || K % kRsK != 0 || log2G < 6 || M < kRsMinM || N < 256 || N % 4 != 0 ||
-      (long long)N * K > 0x7fffffffLL || (long long)M * K > 0x3fffffffLL)
-    return 1;
+  return best;
+}
+
+// The register-stationary kernel takes K % 128 == 0, G >= 64, M >= 33, operands within 31-bit offsets
+bool rs_takes(int M, int N, int K, int log2G) {
+  return K % kRsK == 0 && log2G >= 6 && M >= kRsMinM && N >= 128 && (long long)N * K <= 0x7fffffffLL &&
+         (long long)M * K <= 0x3fffffffLL;
+}
+// unsplit from 160 tiles of 128 x 64 on; below, the wide kernel's 64 x 64 tiles reach more CUs (TinyLlama o and down at
+// M 512: 11.4 and 31.3 us against 13.8 and 34.2 at 128 tiles)
+RsId rs_unsplit(int M, int N, int K, int log2G) {
+  if (!rs_takes(M, N, K, log2G) || (long long)((N + 127) / 128) * ((M + 63) / 64) < 160) return kRsNone;
+  double sc;
+  return rs_best(M, N, 1, &sc).id;
+}
+
+// Split-K (a workspace given, epilogue 0 or 2 = the partials alone): the k ranges S, 1 if the shape does not split. The
+// partials cost traffic (S x M x N x 4 bytes, written and read back) and, unless the next norm sums them, a launch.
+//   * M >= 768: the S in 1, 2, 4 (16 chunks of 128 per range at least) with the best rate over its best tiling, the
+//     partials priced at 800 S / K of the product's time; no split unless 5% better, nor where K is under 64 chunks and
+//     the unsplit kernel has its tiles. 4096 x 14336 at M 2048 228 us unsplit (256 x 128) against 298 split 2 ways over
+//     256 x 64 tiles of four waves, at M 1024 122 split 4 ways over 512 x 128 (125 split 2 ways over 256 x 128) against 148.
+//   * below: when the unsplit kernel lacks its tiles or K has 64 chunks, the smallest power of two that gives 384
+//     workgroups of 256 x 64 (else 128 x 64) while every range keeps 16 chunks, if that reaches 192 (4096 x 14336 at M 512:
+//     S 4; TinyLlama's qkv 2560 x 2048 at S 4, 4 chunks per range: 27 us against 19 unsplit).
+//   * up to 128 tokens the partials are small and the alternative is the wide kernel with a few tiles, so there shorter
+//     ranges (5 chunks) pay while the 128 x 64 tiles alone leave three quarters of the CUs idle: 4096 x 14336 at M 64 20.8 us
+//     against 66.2, 4096 x 4096 at M 33 / 64 / 128 13.0 / 13.6 / 16.3 against 18.9 / 20.5 / 19.9, 2048 x 5632 at 64
+//     12.0 against 26.4; with 96 tiles (6144 x 4096 at M 128) they lose, 21 against 19.2.
+constexpr int kSplitMinChunks = 16;
+int gemm_w4a16_splits(int M, int N, int K, int log2G, int epilogue) {
+  if (epilogue != 0 && epilogue != 2) return 1;
+  if (gemm_thin_fits(M, N, K, log2G)) return gemm_thin_splits(M, N, K, log2G);
+  if (!rs_takes(M, N, K, log2G) || N < 256 || N % 4 != 0) return 1;
   const int nk = K / kRsK;
-  if (nk < 64 && gemm_w4a16_rs_tile(M, N, K, log2G) != 0) return 1;
+  if (nk < 64 && rs_unsplit(M, N, K, log2G) != kRsNone) return 1;
+  if (M >= 768) {
+    int best = 1;
+    double top;
+    rs_best(M, N, 1, &top);
+    top *= 1.05;
+    for (int s = 2; s <= 4 && nk / s >= kSplitMinChunks; s *= 2) {
+      double sc;
+      rs_best(M, N, s, &sc);
+      sc /= 1.0 + 800.0 * s / K;
+      if (sc > top) {
+        top = sc;
+        best = s;
+      }
+    }
+    return best;
+  }
   const long long tm = (M + 63) / 64;
-  for (int r = M < 64 ? 32 : 64; r >= 32; r /= 2) {
-    const long long tiles = (N + 4 * r - 1) / (4 * r) * tm;
+  for (int rows = M < 64 ? 128 : 256; rows >= 128; rows /= 2) {
+    const long long tiles = (N + rows - 1) / rows * tm;
     int s = 2;
     while (s < 16 && tiles * s < 384 && nk / (2 * s) >= kSplitMinChunks) s *= 2;
-    if (nk / s >= kSplitMinChunks && tiles * s >= 192) {
-      *rw = r;
-      return s;
-    }
+    if (nk / s >= kSplitMinChunks && tiles * s >= 192) return s;
   }
   if (M <= 128) {
     const long long tiles = (N + 127) / 128 * tm;
     int s = 2;
     while (s < 16 && tiles * s < 192 && nk / (2 * s) >= 5) s *= 2;
-    if (tiles <= 64 && nk / s >= 5 && tiles * s >= 128) {
-      *rw = 32;
-      return s;
-    }
+    if (tiles <= 64 && nk / s >= 5 && tiles * s >= 128) return s;
   }
   return 1;
 }
 
+void launch_rs_id(RsId id, const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
+                  int epilogue, int splits, void* ws, hipStream_t st) {
+  switch (id) {
+    case kRs512x128: return launch_rs<64, 128, 8>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
+    case kRs256x128: return launch_rs<32, 128, 8>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
+    case kRs256x64: return launch_rs<32, 64, 8>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
+    case kRs256x128w4: return launch_rs<64, 128, 4>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
+    case kRs128x128w4: return launch_rs<32, 128, 4>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
+    default: break;
+  }
+  // fewer than 64 tokens: the tile's rows past M are clamped (28672 x 4096 at M 48: 29.7 us against 46.4 on the wide
+  // kernel, which took these before; up to 32 tokens are gemm_thin.hip's)
+  if (M < 64) return launch_rs<32, 64, 4, true>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
+  launch_rs<32, 64, 4>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
+}
+
+}  // namespace
+
 size_t gemm_w4a16_workspace_bytes(int M, int N, int K, int log2G, int epilogue) {
-  int rw;
-  const int s = gemm_w4a16_splits(M, N, K, log2G, epilogue, &rw);
+  const int s = gemm_w4a16_splits(M, N, K, log2G, epilogue);
   return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
 
-// the unsplit register-stationary tiling (see gemm_w4a16_tile), 0 if none has its tiles
-int gemm_w4a16_rs_tile(int M, int N, int K, int log2G) {
-  if (!DK_GEMM_RS || K % kRsK != 0 || log2G < 6 || (long long)N * K > 0x7fffffffLL || (long long)M * K > 0x3fffffffLL)
-    return 0;
-  // weight tiles of 256 (64 rows per wave) and 128 (32 rows per wave), token tiles of 128 and 64
-  const long long n_t = (N + 255) / 256, n_t32 = (N + 127) / 128, tm128 = (M + 127) / 128, tm64 = (M + 63) / 64;
-  if (M >= 128 && N >= 256 && n_t * tm128 >= 320) return 42;
-  if (M >= 128 && N >= 128 && n_t32 * tm128 >= 320) return 52;
-  if (M >= kRsMinM && N >= 128 && n_t32 * tm64 >= 160) return 51;
-  return 0;
-}
-
+// The wide kernel's tile: the largest of 128 x 128, 128 x 64, 64 x 64 whose grid still covers the 256 CUs, then K groups
+// (KG = 2 or 4 four-wave groups per workgroup; 2 at most for 128 x 64, by LDS) while the grid leaves CUs with a single
+// workgroup (returns 10 * tile + KG, tile 3: 128 x 128, 2: 128 x 64, 1: 64 x 64); K % 64 != 0 takes the 64 x 64
+// 16x16x16 kernel above (returns 0).
 int gemm_w4a16_tile(int M, int N, int K, int log2G) {
   if (K % kWK != 0) return 0;
-  const int rs = gemm_w4a16_rs_tile(M, N, K, log2G);
-  if (rs != 0) return rs;
   const long long t128 = (long long)((M + 127) / 128) * ((N + 127) / 128);
   const long long t64m = (long long)((M + 63) / 64) * ((N + 127) / 128);
   const long long t64 = (long long)((M + 63) / 64) * ((N + 63) / 64);
@@ -856,31 +889,25 @@ int gemm_w4a16_tile(int M, int N, int K, int log2G) {
     tile = 1;
     kgr = t64 > 512 ? 1 : (t64 > 256 ? 2 : 4);
   }
-  if (DK_GEMM_KG > 0 && tile != 3) kgr = tile == 2 ? (DK_GEMM_KG > 2 ? 2 : DK_GEMM_KG) : DK_GEMM_KG;
   while ((K / kWK) % kgr != 0) kgr >>= 1;  // every K group takes the same number of chunks
   return 10 * tile + kgr;
 }
 
 void launch_gemm_w4a16(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
                        int epilogue, void* ws, hipStream_t st) {
-  if (ws != nullptr) {
-    int rw;
-    const int splits = gemm_w4a16_splits(M, N, K, log2G, epilogue, &rw);
-    if (splits > 1) {
-      if (rw == 0) {
-        launch_gemm_thin(packed, sz, x, ws, M, N, K, log2G, 2, splits, st);
-        if (epilogue != 2) launch_splitk_reduce(ws, splits, y, M, N, st);
-        return;
-      }
-      if (rw == 64) return launch_rs<64, 64>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
-      return launch_rs<32, 64>(packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
-    }
+  const int splits = ws != nullptr ? gemm_w4a16_splits(M, N, K, log2G, epilogue) : 1;
+  if (gemm_thin_fits(M, N, K, log2G)) {
+    launch_gemm_thin(packed, sz, x, splits > 1 ? ws : y, M, N, K, log2G, splits > 1 ? 2 : epilogue, splits, st);
+    if (splits > 1 && epilogue != 2) launch_splitk_reduce(ws, splits, y, M, N, st);
+    return;
   }
-  if (gemm_thin_fits(M, N, K, log2G)) return launch_gemm_thin(packed, sz, x, y, M, N, K, log2G, epilogue, 1, st);
+  if (splits > 1) {
+    double sc;
+    return launch_rs_id(rs_best(M, N, splits, &sc).id, packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
+  }
+  const RsId rs = rs_unsplit(M, N, K, log2G);
+  if (rs != kRsNone) return launch_rs_id(rs, packed, sz, x, y, M, N, K, log2G, epilogue, 1, nullptr, st);
   switch (gemm_w4a16_tile(M, N, K, log2G)) {
-    case 42: launch_rs<64, 128>(packed, sz, x, y, M, N, K, log2G, epilogue, 1, nullptr, st); return;
-    case 52: launch_rs<32, 128>(packed, sz, x, y, M, N, K, log2G, epilogue, 1, nullptr, st); return;
-    case 51: launch_rs<32, 64>(packed, sz, x, y, M, N, K, log2G, epilogue, 1, nullptr, st); return;
     case 31: launch_wide<128, 128, 1>(packed, sz, x, y, M, N, K, log2G, epilogue, st); return;
     case 21: launch_wide<128, 64, 1>(packed, sz, x, y, M, N, K, log2G, epilogue, st); return;
     case 22: launch_wide<128, 64, 2>(packed, sz, x, y, M, N, K, log2G, epilogue, st); return;

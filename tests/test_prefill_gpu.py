@@ -208,6 +208,28 @@ def test_gemm_few_tokens_exact_on_integer_grid(K, M, N, Kd, G, S):
         assert_close(act, R.swiglu_ref(torch.cat([want[:, 0::2], want[:, 1::2]], 1)), 1e-3, "swiglu of the exact rows")
 
 
+# the register-stationary tilings with ragged M and N: 512 x 128, 256 x 128 and 256 x 64 in eight waves, 256 x 128,
+# 128 x 128 and 128 x 64 in four; then 512 x 128 over four k ranges of unequal chunks
+@pytest.mark.parametrize("M,N,Kd,S", [(509, 25001, 256, 0), (1030, 5100, 256, 0), (500, 5003, 256, 0),
+                                      (2000, 20002, 128, 0), (1500, 6140, 384, 0), (510, 4100, 128, 0),
+                                      (1021, 4092, 14464, 4)])
+def test_gemm_tilings_exact_on_integer_grid(K, M, N, Kd, S):
+    G = 64
+    packed, sz, wref = _grid_weights(N, Kd, G, seed=M + N + Kd)
+    x = torch.randint(-3, 4, (M, Kd), generator=gen(M + 1)).half()
+    want = (x.float() @ wref.float().t()).half()        # exact sums (multiples of 2^-6 below 2^18), one rounding
+    need = K.gemm_workspace_bytes(M, N, Kd, G)
+    assert need == S * M * N * 4
+    y = torch.full((M, N), 7.0, dtype=torch.half, device=DEV)
+    K.gemm_w4a16(packed, sz, x.to(DEV), y, G,
+                 workspace=torch.full((need,), 0xFF, dtype=torch.uint8, device=DEV) if need else None)
+    assert torch.equal(y.cpu(), want)
+    if N % 2 == 0 and not need:
+        act = torch.full((M, N // 2), 7.0, dtype=torch.half, device=DEV)
+        K.gemm_w4a16(packed, sz, x.to(DEV), act, G, epilogue=1)
+        assert_close(act, R.swiglu_ref(torch.cat([want[:, 0::2], want[:, 1::2]], 1)), 1e-3, "swiglu of the exact rows")
+
+
 @pytest.mark.parametrize("N", [200, 49152])
 def test_gemm_one_hot_rows_exact(K, N):
     """Row i of X is one-hot at k_i, so row i of Y is column k_i of the dequantized weight, bit for bit (N 49152 runs
