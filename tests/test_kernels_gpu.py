@@ -147,6 +147,28 @@ def test_quantize_ties(K):
     assert sz.cpu().float().tolist() == [[[0.5, 1.0]], [[0.5, 0.0]]]
 
 
+@pytest.mark.parametrize("N,Kd,G", [(1, 32, 32), (3, 96, 32), (129, 320, 64), (5, 3200, 128), (7, 1536, 512)])
+@pytest.mark.parametrize("clip", [False, True])
+def test_quantize_ties_and_tails(K, N, Kd, G, clip):
+    """Weights that are small multiples of powers of two (quotients land on ties), a minimum of -0.0, constant and tiny
+    groups, and word counts that end inside a workgroup: codes, scales and zero points (signs of zero included) are the
+    oracle's bits. (The clip factors' errors are sums of few distinct terms here, so the argmin has no near-ties.)"""
+    g = gen(N + Kd)
+    w = torch.randint(-12, 13, (N, Kd), generator=g).half() * torch.pow(2.0, torch.randint(-9, 2, (N, 1), generator=g)).half()
+    w[0, :G // 2] = -0.0
+    w[0, G // 2:G] = w[0, G // 2:G].abs() + 1           # (a group with zeros of both signs has no defined minimum)
+    w[-1, -G:] = 3e-7
+    if N > 2:
+        w[1] = torch.rand(Kd, generator=g).half() + 2.0
+        w[2, ::2] = 0.0
+    packed = torch.full((N, Kd // 8), 7, dtype=torch.int32, device=DEV)
+    sz = torch.empty(N, Kd // G, 2, dtype=torch.half, device=DEV)
+    K.quantize_w4(w.to(DEV), packed, sz, G, clip)
+    q, s, z = Q.quantize(w.numpy(), G, clip)
+    assert np.array_equal(packed.cpu().numpy(), Q.pack(q))
+    assert np.array_equal(sz.cpu().numpy().view(np.uint16), Q.pack_scale_zero(s, z).view(np.uint16))
+
+
 # ---------------------------------------------------------------------------------------------------- attention
 def close_or_rejected(out, ref, tol, what):
     if out is not None:
