@@ -81,7 +81,10 @@ def _check_dtype(t, dtype, name):
 
 
 def _stream(t):
-    return ctypes.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    """The handle of torch's current stream on t's device. As the raw handle (0.08 us): building the Stream object of
+    torch.cuda.current_stream took 2.1 us of an op's 8.5 us of host time, more than half of the smallest GEMV's 2.6 us
+    of GPU time again."""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 class DecodeKernels:

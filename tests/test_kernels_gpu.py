@@ -169,6 +169,27 @@ def test_quantize_ties_and_tails(K, N, Kd, G, clip):
     assert np.array_equal(sz.cpu().numpy().view(np.uint16), Q.pack_scale_zero(s, z).view(np.uint16))
 
 
+def test_ops_launch_on_the_current_stream(K):
+    """The handle that every op passes on is that of torch's current stream, in the main thread and in another, inside
+    and outside a stream context."""
+    import threading
+    from runtime import ext
+    x = torch.empty(1, device=DEV)
+    s = torch.cuda.Stream()
+    seen = []
+
+    def look():
+        seen.append(ext._stream(x) == torch.cuda.current_stream(x.device).cuda_stream)
+        with torch.cuda.stream(s):
+            seen.append(ext._stream(x) == s.cuda_stream and s.cuda_stream != 0)
+
+    look()
+    t = threading.Thread(target=look)
+    t.start()
+    t.join()
+    assert seen == [True] * 4
+
+
 # ---------------------------------------------------------------------------------------------------- attention
 def close_or_rejected(out, ref, tol, what):
     if out is not None:
