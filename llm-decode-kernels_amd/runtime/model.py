@@ -107,6 +107,19 @@ def default_gemv_config(N, K):
     return (3, 2, 16, 1)
 
 
+TUNED_GROUP = 128
+
+
+def for_group(table, group):
+    """A tuning table ("...NxK_G128" -> entry) with entries for `group` too: a shape that was not tuned at this group size
+    takes its entry of G 128. The row tiles follow N, K and the launch, hardly the group, and the defaults are far worse:
+    a decode step of 8 Llama-3-8B layers at context 1000 takes 326 us instead of 377 at G 64, 340 instead of 385 at G 32,
+    315 instead of 373 at G 256 (318 at G 128); 12 TinyLlama layers 283 instead of 297 at G 64."""
+    suffix = f"_G{TUNED_GROUP}"
+    borrowed = {k[: -len(suffix)] + f"_G{group}": v for k, v in table.items() if k.endswith(suffix)}
+    return {**borrowed, **table}
+
+
 class Linear:
     """One projection in the format the config asks for (runtime/model.py:56-72).
 
@@ -221,14 +234,14 @@ class Model:
         self.step_cfg_override = {}
         if cfg.gemv_stage is None and Path(cfg.autotune_path).exists():
             tab = json.load(open(cfg.autotune_path))
-            self.gemv_table = tab.get("best", {})
-            self.gemv_norm_table = tab.get("best_norm", {})
-            self.gemv_us, self.gemv_norm_us = tab.get("us", {}), tab.get("us_norm", {})
-            self.gemv_gate_up_table = tab.get("best_gate_up", {})
+            t = lambda key: for_group(tab.get(key, {}), cfg.group)
+            self.gemv_table, self.gemv_norm_table = t("best"), t("best_norm")
+            self.gemv_us, self.gemv_norm_us = t("us"), t("us_norm")
+            self.gemv_gate_up_table = t("best_gate_up")
             self.gemv_f16_table = tab.get("best_f16", {})
             self.gemv_f16_norm_table = tab.get("best_f16_norm", {})
             # configurations chosen by the decode step time (runtime.autotune.tune_step), ahead of the isolated tables
-            self.step_cfg_override = {k: tuple(v) for k, v in tab.get("best_step", {}).items()}
+            self.step_cfg_override = {k: tuple(v) for k, v in t("best_step").items()}
 
         # paged KV cache [L, 2, pages, n_kv, P, D]; one block table shared by all layers (one sequence)
         self.n_pages = (cfg.max_ctx + cfg.page - 1) // cfg.page + 1

@@ -90,3 +90,13 @@ def test_rope_theta_from_hf_configs():
         return
     assert rope_theta_of(LlamaConfig(rope_theta=500000.0)) == 500000.0
     assert rope_theta_of(LlamaConfig()) == 10000.0
+
+
+def test_untuned_group_borrows_the_entries_of_g128():
+    """Shapes tuned at another group size serve a group without an entry of its own; its own entries win."""
+    from runtime.model import for_group
+    tab = {"2048x2048_G128": [4, 2, 0, 1], "rope:6144x4096_G128": [4, 4, 4, 2], "2048x2048_G64": [3, 2, 1, 0],
+           "f16_norm:32000x2048": [1, 1, 0]}
+    assert for_group(tab, 128) == tab
+    assert for_group(tab, 64) == {**tab, "rope:6144x4096_G64": [4, 4, 4, 2]}
+    assert for_group(tab, 32)["2048x2048_G32"] == [4, 2, 0, 1] and for_group({}, 64) == {}
