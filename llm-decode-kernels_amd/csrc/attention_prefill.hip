@@ -14,11 +14,13 @@
 //     output all live in the lane pair (r, r + 32), so the softmax needs one exchange per block and the output's
 //     rescale factor is the lane's own.
 //   * online softmax in the log2 domain (the scale and log2 e in one multiplier). The reference maximum of a column
-//     moves only when a block's maximum passes it by more than kLazy (2^8): until then p = 2^(s - ref) is at most 2^8,
-//     in range for every type it meets, and neither the accumulators nor the sum need rescaling. Each column decides
+//     moves only when a block's maximum passes it by more than kLazy (2^8); until then neither the accumulators nor the
+//     sum need rescaling. p = 2^(s - ref + kLift), at most 2^15: fp16 holds it, and what its two fp16 parts round away
+//     (2^-25 at most, below 2^-14 a fixed amount) is 2^-32 or less of the largest weight. Each column decides
 //     for itself (the wave only skips the code when none of its columns moves), so a row's result does not depend on
 //     the rows it shares a wave with. Blocks wholly visible to the wave skip the causal mask.
-//   * O^T += V^T . P^T with p as fp16 hi + lo parts (about 22 bits): the score accumulator is the B operand as it is
+//   * O^T += V^T . P^T with p as fp16 hi + lo parts, both rounded to nearest (22 bits, no bias: the sum of the weights
+//     is taken from the unsplit p, so a truncated p lowers every output): the score accumulator is the B operand as it is
 //     (k slot e of half h in step s is token 16 s + 8 (e / 4) + 4 h + e % 4, for both operands), and the V^T operand
 //     comes out of the row-major V tile through the transposing LDS read (ds_read_b64_tr_b16: 4 tokens x 16 dims per 16
 //     lanes, lane i receiving dim i).
@@ -44,8 +46,12 @@ namespace {
 // 2^(score - ref) never meet -inf - (-inf).
 constexpr float kPfNoMax = -1e30f;
 constexpr float kLazy = 8.0f;  // log2 units
+constexpr float kLift = 7.0f;  // p's exponent at the reference maximum
+static_assert(kLazy + kLift <= 15.0f, "p fits fp16");
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef float f2 __attribute__((ext_vector_type(2)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 
@@ -244,12 +250,13 @@ attn_prefill_kernel(const f16* __restrict__ qkv, const int32_t* __restrict__ pos
         for (int i = 0; i < 16; ++i) acc[t][i] *= alpha;
       }
     }
+    const float lift = kLift - mref;
     float ps[2] = {0.f, 0.f};
 #pragma unroll
     for (int tt = 0; tt < NT; ++tt) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        const float p = __builtin_amdgcn_exp2f(fmaf(sc[tt][i], c2, -mref));
+        const float p = __builtin_amdgcn_exp2f(fmaf(sc[tt][i], c2, lift));
         sc[tt][i] = p;
         ps[i & 1] += p;
       }
@@ -261,9 +268,9 @@ attn_prefill_kernel(const f16* __restrict__ qkv, const int32_t* __restrict__ pos
 #pragma unroll
       for (int e = 0; e < 8; e += 2) {
         const float p0 = sc[ks >> 1][8 * (ks & 1) + e], p1 = sc[ks >> 1][8 * (ks & 1) + e + 1];
-        const auto hi = __builtin_amdgcn_cvt_pkrtz(p0, p1);
+        const h2 hi = __builtin_convertvector(f2{p0, p1}, h2);
         const uint32_t hw = __builtin_bit_cast(uint32_t, hi);
-        const auto lo = __builtin_amdgcn_cvt_pkrtz(minus_lo(p0, hw), minus_hi(p1, hw));
+        const h2 lo = __builtin_convertvector(f2{minus_lo(p0, hw), minus_hi(p1, hw)}, h2);
         phi[e] = hi[0];
         phi[e + 1] = hi[1];
         plo[e] = lo[0];

@@ -425,6 +425,32 @@ def test_attention_prefill_workgroup_shapes(K, D, n_q, n_kv, page, start, M):
         assert_close(out[m].view(n_q, D), ref, 2e-3, f"row {m} vs oracle")
 
 
+# one and four groups over the token blocks at each head dim (up to 512 / 256 column waves: four; from 1537 / 4096: one)
+@pytest.mark.parametrize("D,n_kv,start,M", [(64, 4, 4056, 40), (64, 4, 2496, 1600), (64, 4, 16344, 40), (64, 4, 14784, 1600),
+                                            (128, 8, 4056, 40), (128, 8, 0, 4100), (128, 8, 16344, 40), (128, 8, 12284, 4100)])
+@pytest.mark.parametrize("mu", [-12.0, -14.0])
+def test_attention_prefill_sink_token(K, D, n_kv, start, M, mu):
+    """One early token takes most of the weight and thousands share the rest, each with a weight far below 2^-11 of the
+    largest, over values of non-zero mean: what rounding does to the small weights adds up. Each output against float64
+    within 5e-4 of itself: half an fp16 ulp (2^-11 = 4.88e-4) and fp32 sums (1e-5)."""
+    page, n_q = 16, 32
+    kc, vc, bt = make_cache(start + M, n_kv, page, D=D, seed=M)
+    g = gen(int(-mu) + start)
+    kc[..., 0] = ((mu + 1.5 * torch.randn(kc.shape[:3], generator=g)) * D ** 0.5 / 8).half()
+    vc.mul_(0.1).add_(1.0)
+    kc[int(bt[0]), :, 0, 0] = 0.0                       # token 0: score 0
+    vc[int(bt[0]), :, 0] = 0.05
+    qkv = torch.zeros(M, (n_q + 2 * n_kv) * D, dtype=torch.half)
+    qkv[:, : n_q * D : D] = 8.0
+    out = _prefill_attn(K, qkv, start, kc.to(DEV), vc.to(DEV), bt.to(DEV), n_q, n_kv, start + M).double().cpu()
+    k, v = (t.double() for t in R.gather_kv(kc, vc, bt, start + M, page))       # [ctx, n_kv, D]
+    for m in sorted({M - 1, M // 2, M // 7, 3}):
+        p = torch.softmax(k[: start + m + 1, :, 0] * 8.0 / D ** 0.5, 0)
+        want = (p.unsqueeze(-1) * v[: start + m + 1]).sum(0).repeat_interleave(n_q // n_kv, 0)
+        err = (out[m].view(n_q, D) / want - 1).abs().max()
+        assert err < 5e-4, (m, float(err))
+
+
 @pytest.mark.parametrize("D,M", [(64, 40), (64, 1700), (128, 300), (128, 1700)])
 def test_attention_prefill_unmapped_page_reads_zeros(K, D, M):
     """A block-table entry outside the cache gives zero K / V rows: the same bits as a page of zeros; an output that is
