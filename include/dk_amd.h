@@ -202,12 +202,17 @@ int dk_gemm_w4a16(const void* packed, const void* sz, const void* x, void* y, in
  * N] to the workspace and sum them in a second launch, in split order (the result does not depend on scheduling; its
  * fp32 summation order differs from the unsplit kernel's). dk_gemm_w4a16_workspace_bytes returns the bytes a shape
  * needs (0: it does not split; epilogue 1 never splits); the bytes do not grow steadily with M, so one buffer for
- * several M takes the largest of their answers. workspace NULL runs dk_gemm_w4a16; otherwise it must hold that many
- * bytes, be 16-byte aligned and overlap neither x nor y. epilogue 2 (shapes that split only; y unused, may be NULL):
- * the partials alone, left in the workspace for a reader that sums them (dk_rmsnorm_rows_parts), which saves the
- * second launch. Like dk_gemm_w4a16, no counterpart in the reference.
+ * several M takes the largest of their answers. workspace NULL runs dk_gemm_w4a16; otherwise it must be 16-byte aligned
+ * and overlap neither x nor y. A smaller workspace runs the most k ranges that it holds (half or a quarter of them and
+ * so on), or none, where the split is a matter of speed alone (up to 128 tokens, or from 768 on, mostly); where the
+ * weight rows leave CUs idle at M >= 64 and K has 16 chunks of 128 for every range, it is refused (DK_ERR_SHAPE).
+ * epilogue 2 (shapes that split only; y unused, may be NULL): the partials alone, left in the workspace for a reader
+ * that sums them (dk_rmsnorm_rows_parts), which saves the second launch; it takes the whole workspace.
+ * dk_gemm_w4a16_ws_splits says what a call does: the k ranges it runs over with a workspace of that many bytes (1: it
+ * does not split), 0 where it refuses. Like dk_gemm_w4a16, no counterpart in the reference.
  */
 size_t dk_gemm_w4a16_workspace_bytes(int M, int N, int K, int group, int epilogue);
+int dk_gemm_w4a16_ws_splits(int M, int N, int K, int group, int epilogue, size_t workspace_bytes);
 int dk_gemm_w4a16_ws(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int group,
                      int epilogue, void* workspace, size_t workspace_bytes, void* stream);
 

@@ -260,13 +260,26 @@ int dk_gemm_w4a16(const void* packed, const void* sz, const void* x, void* y, in
   const int rc = gemm_check(packed, sz, x, y, M, N, K, group, epilogue);
   if (rc != DK_OK) return rc;
   clear_error();
-  dk::launch_gemm_w4a16(packed, sz, x, y, M, N, K, ilog2(group), epilogue, nullptr, (hipStream_t)stream);
+  dk::launch_gemm_w4a16(packed, sz, x, y, M, N, K, ilog2(group), epilogue, 1, nullptr,
+                        (hipStream_t)stream);
   return launched("gemm_w4a16");
 }
 
 size_t dk_gemm_w4a16_workspace_bytes(int M, int N, int K, int group, int epilogue) {
   if (M <= 0 || N <= 0 || K <= 0 || group < 32 || !pow2(group) || K % group != 0) return 0;
-  return dk::gemm_w4a16_workspace_bytes(M, N, K, ilog2(group), epilogue);
+  const int s = dk::gemm_w4a16_splits(M, N, K, ilog2(group), epilogue);
+  return s > 1 ? (size_t)s * M * N * sizeof(float) : 0;
+}
+
+int dk_gemm_w4a16_ws_splits(int M, int N, int K, int group, int epilogue, size_t workspace_bytes) {
+  const size_t need = dk_gemm_w4a16_workspace_bytes(M, N, K, group, epilogue);
+  if (need == 0) return epilogue == 2 ? 0 : 1;
+  const size_t range = (size_t)M * N * sizeof(float);
+  const int least = dk::gemm_w4a16_min_splits(M, N, K, ilog2(group), epilogue);
+  if (least > 1 && workspace_bytes < least * range) return 0;
+  int s = (int)(need / range);
+  while (s > 1 && workspace_bytes < s * range) s >>= 1;
+  return s;
 }
 
 int dk_gemm_w4a16_ws(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int group,
@@ -274,22 +287,27 @@ int dk_gemm_w4a16_ws(const void* packed, const void* sz, const void* x, void* y,
   const bool parts = epilogue == 2;  // the fp32 split partials alone, left in the workspace (y unused)
   const int rc = gemm_check(packed, sz, x, parts ? workspace : y, M, N, K, group, parts ? 0 : epilogue);
   if (rc != DK_OK) return rc;
-  const size_t need = dk::gemm_w4a16_workspace_bytes(M, N, K, ilog2(group), epilogue);
+  const size_t need = dk_gemm_w4a16_workspace_bytes(M, N, K, group, epilogue);
   if (parts && need == 0)
     return fail(DK_ERR_DOMAIN, "gemm_w4a16_ws: epilogue 2 (split partials only) needs a shape that splits "
                                "(gemm_w4a16_workspace_bytes > 0)");
+  int splits = 1;
   if (workspace != nullptr) {
-    if (workspace_bytes < need)
+    splits = dk_gemm_w4a16_ws_splits(M, N, K, group, epilogue, workspace_bytes);
+    if (splits == 0)
       return fail(DK_ERR_SHAPE, "gemm_w4a16_ws: workspace of %zu bytes, this shape needs %zu", workspace_bytes, need);
     if (!aligned16(workspace)) return fail(DK_ERR_ALIGN, "gemm_w4a16_ws: workspace must be 16B aligned");
-    if (!parts && need > 0 && ranges_overlap(workspace, need, y, (size_t)M * N * 2))
-      return fail(DK_ERR_DOMAIN, "gemm_w4a16_ws: workspace must not overlap y");
-    if (need > 0 && ranges_overlap(workspace, need, x, (size_t)M * K * 2))
-      return fail(DK_ERR_DOMAIN, "gemm_w4a16_ws: workspace must not overlap x");
+    const size_t used = splits > 1 ? (size_t)splits * M * N * sizeof(float) : 0;
+    const bool on_y = !parts && used > 0 && ranges_overlap(workspace, used, y, (size_t)M * N * 2);
+    const bool on_x = used > 0 && ranges_overlap(workspace, used, x, (size_t)M * K * 2);
+    if (on_y || on_x) {
+      if (dk::gemm_w4a16_min_splits(M, N, K, ilog2(group), epilogue) > 1)
+        return fail(DK_ERR_DOMAIN, "gemm_w4a16_ws: workspace must not overlap %s", on_y ? "y" : "x");
+      splits = 1;  // a workspace that the shape can do without
+    }
   }
   clear_error();
-  dk::launch_gemm_w4a16(packed, sz, x, y, M, N, K, ilog2(group), epilogue, need > 0 ? workspace : nullptr,
-                        (hipStream_t)stream);
+  dk::launch_gemm_w4a16(packed, sz, x, y, M, N, K, ilog2(group), epilogue, splits, workspace, (hipStream_t)stream);
   return launched("gemm_w4a16_ws");
 }
 

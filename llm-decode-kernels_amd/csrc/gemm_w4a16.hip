@@ -808,42 +808,22 @@ RsId rs_unsplit(int M, int N, int K, int log2G) {
 //     against 66.2, 4096 x 4096 at M 33 / 64 / 128 13.0 / 13.6 / 16.3 against 18.9 / 20.5 / 19.9, 2048 x 5632 at 64
 //     12.0 against 26.4; with 96 tiles (6144 x 4096 at M 128) they lose, 21 against 19.2.
 constexpr int kSplitMinChunks = 16;
-int gemm_w4a16_splits(int M, int N, int K, int log2G, int epilogue) {
-  if (epilogue != 0 && epilogue != 2) return 1;
-  if (gemm_thin_fits(M, N, K, log2G)) return gemm_thin_splits(M, N, K, log2G);
-  if (!rs_takes(M, N, K, log2G) || N < 256 || N % 4 != 0) return 1;
+
+// the second rule, without a bound on M: 1 if it does not split
+int base_splits(int M, int N, int K, int log2G, int max_rows) {
   const int nk = K / kRsK;
   if (nk < 64 && rs_unsplit(M, N, K, log2G) != kRsNone) return 1;
-  if (M >= 768) {
-    int best = 1;
-    double top;
-    rs_best(M, N, 1, &top);
-    top *= 1.05;
-    for (int s = 2; s <= 4 && nk / s >= kSplitMinChunks; s *= 2) {
-      double sc;
-      rs_best(M, N, s, &sc);
-      sc /= 1.0 + 800.0 * s / K;
-      if (sc > top) {
-        top = sc;
-        best = s;
-      }
-    }
-    return best;
-  }
   const long long tm = (M + 63) / 64;
-  for (int rows = M < 64 ? 128 : 256; rows >= 128; rows /= 2) {
+  for (int rows = max_rows; rows >= 128; rows /= 2) {
     const long long tiles = (N + rows - 1) / rows * tm;
     int s = 2;
     while (s < 16 && tiles * s < 384 && nk / (2 * s) >= kSplitMinChunks) s *= 2;
     if (nk / s >= kSplitMinChunks && tiles * s >= 192) return s;
   }
-  if (M <= 128) {
-    const long long tiles = (N + 127) / 128 * tm;
-    int s = 2;
-    while (s < 16 && tiles * s < 192 && nk / (2 * s) >= 5) s *= 2;
-    if (tiles <= 64 && nk / s >= 5 && tiles * s >= 128) return s;
-  }
   return 1;
+}
+bool may_split(int M, int N, int K, int log2G, int epilogue) {
+  return (epilogue == 0 || epilogue == 2) && N >= 256 && N % 4 == 0 && rs_takes(M, N, K, log2G);
 }
 
 void launch_rs_id(RsId id, const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
@@ -864,9 +844,47 @@ void launch_rs_id(RsId id, const void* packed, const void* sz, const void* x, vo
 
 }  // namespace
 
-size_t gemm_w4a16_workspace_bytes(int M, int N, int K, int log2G, int epilogue) {
+int gemm_w4a16_splits(int M, int N, int K, int log2G, int epilogue) {
+  if ((epilogue == 0 || epilogue == 2) && gemm_thin_fits(M, N, K, log2G)) return gemm_thin_splits(M, N, K, log2G);
+  if (!may_split(M, N, K, log2G, epilogue)) return 1;
+  const int nk = K / kRsK;
+  if (M >= 768) {
+    if (nk < 64 && rs_unsplit(M, N, K, log2G) != kRsNone) return 1;
+    int best = 1;
+    double top;
+    rs_best(M, N, 1, &top);
+    top *= 1.05;
+    for (int s = 2; s <= 4 && nk / s >= kSplitMinChunks; s *= 2) {
+      double sc;
+      rs_best(M, N, s, &sc);
+      sc /= 1.0 + 800.0 * s / K;
+      if (sc > top) {
+        top = sc;
+        best = s;
+      }
+    }
+    return best;
+  }
+  const int base = base_splits(M, N, K, log2G, M < 64 ? 128 : 256);
+  if (base > 1 || (nk < 64 && rs_unsplit(M, N, K, log2G) != kRsNone)) return base;
+  if (M <= 128) {
+    const long long tiles = (long long)((N + 127) / 128) * ((M + 63) / 64);
+    int s = 2;
+    while (s < 16 && tiles * s < 192 && nk / (2 * s) >= 5) s *= 2;
+    if (tiles <= 64 && nk / s >= 5 && tiles * s >= 128) return s;
+  }
+  return 1;
+}
+
+// Shapes of M >= 64 that the base rule splits need a workspace of that many k ranges at least (a smaller one is a wrong
+// size); for the others a workspace is an offer, and one that holds fewer ranges than gemm_w4a16_splits is used for
+// what it holds.
+int gemm_w4a16_min_splits(int M, int N, int K, int log2G, int epilogue) {
   const int s = gemm_w4a16_splits(M, N, K, log2G, epilogue);
-  return s > 1 ? (size_t)s * (size_t)M * (size_t)N * sizeof(float) : 0;
+  if (epilogue == 2 || s == 1) return s;  // the reader of the partials counts on all of them
+  if (M < 64 || !may_split(M, N, K, log2G, epilogue)) return 1;
+  const int base = base_splits(M, N, K, log2G, 256);
+  return base < s ? base : s;
 }
 
 // The wide kernel's tile: the largest of 128 x 128, 128 x 64, 64 x 64 whose grid still covers the 256 CUs, then K groups
@@ -894,8 +912,7 @@ int gemm_w4a16_tile(int M, int N, int K, int log2G) {
 }
 
 void launch_gemm_w4a16(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
-                       int epilogue, void* ws, hipStream_t st) {
-  const int splits = ws != nullptr ? gemm_w4a16_splits(M, N, K, log2G, epilogue) : 1;
+                       int epilogue, int splits, void* ws, hipStream_t st) {
   if (gemm_thin_fits(M, N, K, log2G)) {
     launch_gemm_thin(packed, sz, x, splits > 1 ? ws : y, M, N, K, log2G, splits > 1 ? 2 : epilogue, splits, st);
     if (splits > 1 && epilogue != 2) launch_splitk_reduce(ws, splits, y, M, N, st);

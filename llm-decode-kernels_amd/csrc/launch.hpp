@@ -71,11 +71,13 @@ void launch_gemv_f16(int prologue, int R, int waves, int pf, const void* w, cons
                      int K, hipStream_t st);
 
 // W4A16 GEMM (prefill): Y[M, N] = X[M, K] . dequant(W)^T; epilogue 1 = SwiGLU of interleaved gate/up column pairs
-// (Y [M, N/2]). K % 32 == 0, group >= 32.
+// (Y [M, N/2]). K % 32 == 0, group >= 32. splits > 1: over that many k ranges, fp32 partials [splits, M, N] in ws.
 void launch_gemm_w4a16(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
-                       int epilogue, void* ws, hipStream_t st);
-// bytes of fp32 split-K partials launch_gemm_w4a16 uses for this shape when given a workspace (0: it does not split)
-size_t gemm_w4a16_workspace_bytes(int M, int N, int K, int log2G, int epilogue);
+                       int epilogue, int splits, void* ws, hipStream_t st);
+// the k ranges a shape splits into when its workspace holds them all (a power of two, 1: it does not split), and the
+// fewest that a workspace must hold
+int gemm_w4a16_splits(int M, int N, int K, int log2G, int epilogue);
+int gemm_w4a16_min_splits(int M, int N, int K, int log2G, int epilogue);
 
 // The GEMM of a few tokens (gemm_thin.hip): whether a shape takes it, the k ranges it splits into when a workspace is
 // given (1: it does not split), and its launch (splits > 1: y receives the fp32 partials [splits, M, N]).

@@ -33,6 +33,7 @@ SIGNATURES = {
     "dk_gemv_f16_rmsnorm": ([_I, _I, _I, _P, _P, _P, _P, _F, _P, _P, _I, _I, _P], _I),
     "dk_gemm_w4a16": ([_P, _P, _P, _P, _I, _I, _I, _I, _I, _P], _I),
     "dk_gemm_w4a16_workspace_bytes": ([_I, _I, _I, _I, _I], _Z),
+    "dk_gemm_w4a16_ws_splits": ([_I, _I, _I, _I, _I, _Z], _I),
     "dk_gemm_w4a16_ws": ([_P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _Z, _P], _I),
     "dk_rope_append_rows": ([_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P], _I),
     "dk_rmsnorm_rows_parts": ([_P, _P, _I, ctypes.c_longlong, _P, _P, _P, _I, _I, _F, _P], _I),
@@ -269,8 +270,8 @@ class DecodeKernels:
         return int(self.lib.dk_gemm_w4a16_workspace_bytes(int(M), int(N), int(K), int(group), int(epilogue)))
 
     def gemm_w4a16(self, packed, sz, x, y, group, epilogue=0, workspace=None):
-        """y = x . dequant(W)^T (epilogue 1: SwiGLU of interleaved gate/up rows); `workspace` (a CUDA tensor of at
-        least gemm_workspace_bytes bytes) lets the shapes that do not fill the CUs split K."""
+        """y = x . dequant(W)^T (epilogue 1: SwiGLU of interleaved gate/up rows); `workspace` (a CUDA tensor of
+        gemm_workspace_bytes bytes) lets the shapes that do not fill the CUs split K."""
         for t, n in ((packed, "packed"), (sz, "sz"), (x, "x"), (y, "y")):
             _check_cuda(t, n)
         N, K = packed.size(0), packed.size(1) * 8

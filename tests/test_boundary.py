@@ -284,6 +284,27 @@ def test_small_op_validation(lib):
     assert bw(n=8)[0] == 3 and bw(sink=None)[0] == 1 and bw(buf=None)[0] == 1
 
 
+@pytest.mark.parametrize("M,N,K,S,least", [
+    (16, 4096, 14336, 8, 1), (33, 4096, 4096, 4, 1), (64, 4096, 4096, 4, 1), (128, 2048, 5632, 8, 1),   # up to 128 tokens
+    (512, 4096, 14336, 4, 4), (512, 2048, 5632, 2, 2), (767, 4096, 14336, 2, 2),                        # idle CUs, long k
+    (1000, 4096, 14336, 4, 2)])
+def test_gemm_workspace_smaller_than_the_need(lib, M, N, K, S, least):
+    """A workspace that holds fewer than the S ranges of a shape runs the largest power of two it holds, down to none
+    where the split is a matter of speed; a shape that needs `least` ranges refuses fewer. The partials alone
+    (epilogue 2) take them all."""
+    part = M * N * 4
+    assert lib.dk_gemm_w4a16_workspace_bytes(M, N, K, 128, 0) == S * part
+    for held in (0, 1, part - 1, part, 2 * part - 1, 2 * part, 3 * part, 4 * part - 1, 4 * part, 8 * part):
+        whole = min(held // part, S)
+        want = 1 << (whole.bit_length() - 1) if whole > 1 else 1
+        want = 0 if least > 1 and whole < least else want
+        assert lib.dk_gemm_w4a16_ws_splits(M, N, K, 128, 0, held) == want, held
+        assert lib.dk_gemm_w4a16_ws_splits(M, N, K, 128, 1, held) == 1
+        assert lib.dk_gemm_w4a16_ws_splits(M, N, K, 128, 2, held) == (S if whole == S else 0)
+    assert lib.dk_gemm_w4a16_ws_splits(512, 4096, 4096, 128, 0, 1 << 30) == 1
+    assert lib.dk_gemm_w4a16_ws_splits(512, 4096, 4096, 128, 2, 1 << 30) == 0
+
+
 def test_prefill_validation(lib):
     g = lambda **kw: _err(lib, lib.dk_gemm_w4a16(*dict(dict(p=A16, sz=A16, x=A16, y=B16, M=64, N=128, K=256, G=128,
                                                             epi=0), **kw).values(), None))

@@ -179,6 +179,31 @@ def test_gemm_splitk_one_hot_rows_exact(K):
     assert torch.equal(y.cpu(), wref[:, ks].t().contiguous())
 
 
+@pytest.mark.parametrize("M,N,Kd", [(16, 4096, 14336), (33, 4096, 4096), (100, 2048, 5632), (1000, 4096, 14336)])
+def test_gemm_smaller_workspace_runs_what_it_holds(K, M, N, Kd):
+    """A workspace of fewer ranges than the shape splits into is used for the power of two it holds (exact on the integer
+    grid, nothing written past it); one that lies over x is left alone where the shape can do without."""
+    G, part = 128, M * N * 4
+    packed, sz, wref = _grid_weights(N, Kd, G, seed=M + Kd)
+    x = torch.randint(-3, 4, (M, Kd), generator=gen(M)).half()
+    want = (x.double() @ wref.double().t()).half()
+    need = K.gemm_workspace_bytes(M, N, Kd, G)
+    least = 2 * part if M >= 768 else 16
+    buf = torch.empty(need + x.numel() * 2, dtype=torch.uint8, device=DEV)
+    for held in sorted({least, need // 2, need // 2 + 16, need - 16, need} | ({part} if least == 16 else set())):
+        buf.fill_(0xA5)
+        y = torch.full((M, N), 7.0, dtype=torch.half, device=DEV)
+        K.gemm_w4a16(packed, sz, x.to(DEV), y, G, workspace=buf[:held])
+        assert torch.equal(y.cpu(), want), held
+        assert bool((buf[held:] == 0xA5).all()), held
+    if least == 16:
+        xb = buf[: x.numel() * 2].view(torch.half).view(M, Kd)
+        xb.copy_(x)
+        y = torch.full((M, N), 7.0, dtype=torch.half, device=DEV)
+        K.gemm_w4a16(packed, sz, xb, y, G, workspace=buf)
+        assert torch.equal(y.cpu(), want) and torch.equal(xb.cpu(), x)
+
+
 # few tokens: the thin kernel at 128, 64, 32 and 16 weight rows per workgroup (ragged N, K not a multiple of 256, more
 # chunks than groups by a remainder, so that some groups end on a chunk of zeros) and its split-K; the 64-token
 # register-stationary tile with fewer tokens, unsplit and split, and short splits up to 128 tokens
