@@ -15,7 +15,7 @@
 // reference sums them in fp32, so the two can pick different factors only where two errors agree to fp32 summation
 // noise.
 //
-// One lane per packed word (8 weights, one 16-byte load), kWordsPerThread words per thread; the G/8 lanes of a group are
+// One lane per packed word (8 weights, one 16-byte load), 1 or 4 words per thread (kManyWords); the G/8 lanes of a group are
 // consecutive in one wave (G <= 512) and reduce min / max (and the clip errors) by DPP within 16 lanes, by shuffles
 // beyond. Rows are whole groups, so words and groups are numbered through the matrix and no row is ever computed.
 // Bound: the 2.5 bytes per weight. Before, the row's 64-bit division, ten IEEE divisions per word and eight LDS
@@ -99,18 +99,18 @@ __device__ __forceinline__ void group_total(double& e) {
   }
 }
 
-constexpr int kWordsPerThread = 4, kQuantThreads = 256;
+constexpr int kQuantThreads = 256;
 
-template <int WPG, bool CLIP>  // words (lanes) per group; range clipping
+template <int WPG, bool CLIP, int WPT>  // words (lanes) per group; range clipping; words per thread
 __global__ void __launch_bounds__(kQuantThreads)
 quantize_w4_kernel(const f16* __restrict__ w, uint32_t* __restrict__ packed, uint32_t* __restrict__ sz, long long words) {
-  const long long base = (long long)blockIdx.x * (kQuantThreads * kWordsPerThread) + threadIdx.x;
-  u32x4 raw[kWordsPerThread];
+  const long long base = (long long)blockIdx.x * (kQuantThreads * WPT) + threadIdx.x;
+  u32x4 raw[WPT];
 #pragma unroll
-  for (int i = 0; i < kWordsPerThread; ++i)  // dead tail lanes (whole dead groups: words % WPG == 0) re-read the last word
+  for (int i = 0; i < WPT; ++i)  // dead tail lanes (whole dead groups: words % WPG == 0) re-read the last word
     raw[i] = load_stream(reinterpret_cast<const u32x4*>(w) + min(base + i * kQuantThreads, words - 1));
 #pragma unroll
-  for (int i = 0; i < kWordsPerThread; ++i) {
+  for (int i = 0; i < WPT; ++i) {
     const long long gid = base + i * kQuantThreads;
     float v[8];
     unpack8(raw[i], v);
@@ -176,30 +176,38 @@ quantize_w4_kernel(const f16* __restrict__ w, uint32_t* __restrict__ packed, uin
   }
 }
 
-template <bool CLIP>
+// Words per thread: a thread works through its words one after the other, so where the waves are few the chain of four is
+// the kernel's time; over many rounds of waves four loads in flight per thread are a little better. us at G 128 with 1 / 4
+// words (clip: 1 / 4): 256 x 1024 2.8 / 3.6 (6.0 / 18.2), 1024 x 4096 4.5 / 4.8 (15.7 / 21.5), 4096 x 4096 11.9 / 11.9 (51.5 /
+// 54.7), 4096 x 14336 33.5 / 33.7 (167 / 166), 16384 x 14336 125 / 119 (648 / 628).
+constexpr long long kManyWords = 1 << 22;
+
+template <bool CLIP, int WPT>
 void launch_quantize(const void* w, void* packed, void* sz, int N, int K, int log2G, hipStream_t st) {
   const long long words = (long long)N * (K >> 3);
-  const int per = kQuantThreads * kWordsPerThread;
+  const int per = kQuantThreads * WPT;
   const dim3 grid((unsigned)((words + per - 1) / per)), block(kQuantThreads);
   const f16* wp = (const f16*)w;
   uint32_t* pp = (uint32_t*)packed;
   uint32_t* sp = (uint32_t*)sz;
   switch (log2G) {
-    case 5: hipLaunchKernelGGL((quantize_w4_kernel<4, CLIP>), grid, block, 0, st, wp, pp, sp, words); break;
-    case 6: hipLaunchKernelGGL((quantize_w4_kernel<8, CLIP>), grid, block, 0, st, wp, pp, sp, words); break;
-    case 7: hipLaunchKernelGGL((quantize_w4_kernel<16, CLIP>), grid, block, 0, st, wp, pp, sp, words); break;
-    case 8: hipLaunchKernelGGL((quantize_w4_kernel<32, CLIP>), grid, block, 0, st, wp, pp, sp, words); break;
-    default: hipLaunchKernelGGL((quantize_w4_kernel<64, CLIP>), grid, block, 0, st, wp, pp, sp, words); break;
+    case 5: hipLaunchKernelGGL((quantize_w4_kernel<4, CLIP, WPT>), grid, block, 0, st, wp, pp, sp, words); break;
+    case 6: hipLaunchKernelGGL((quantize_w4_kernel<8, CLIP, WPT>), grid, block, 0, st, wp, pp, sp, words); break;
+    case 7: hipLaunchKernelGGL((quantize_w4_kernel<16, CLIP, WPT>), grid, block, 0, st, wp, pp, sp, words); break;
+    case 8: hipLaunchKernelGGL((quantize_w4_kernel<32, CLIP, WPT>), grid, block, 0, st, wp, pp, sp, words); break;
+    default: hipLaunchKernelGGL((quantize_w4_kernel<64, CLIP, WPT>), grid, block, 0, st, wp, pp, sp, words); break;
   }
 }
 
 }  // namespace
 
 void launch_quantize_w4(const void* w, void* packed, void* sz, int N, int K, int log2G, int clip, hipStream_t st) {
-  if (clip)
-    launch_quantize<true>(w, packed, sz, N, K, log2G, st);
-  else
-    launch_quantize<false>(w, packed, sz, N, K, log2G, st);
+  if ((long long)N * (K >> 3) > kManyWords) {
+    if (clip) return launch_quantize<true, 4>(w, packed, sz, N, K, log2G, st);
+    return launch_quantize<false, 4>(w, packed, sz, N, K, log2G, st);
+  }
+  if (clip) return launch_quantize<true, 1>(w, packed, sz, N, K, log2G, st);
+  launch_quantize<false, 1>(w, packed, sz, N, K, log2G, st);
 }
 
 }  // namespace dk

@@ -169,6 +169,25 @@ def test_quantize_ties_and_tails(K, N, Kd, G, clip):
     assert np.array_equal(sz.cpu().numpy().view(np.uint16), Q.pack_scale_zero(s, z).view(np.uint16))
 
 
+@pytest.mark.parametrize("G", [32, 128, 512])
+@pytest.mark.parametrize("clip", [False, True])
+def test_quantize_large_equals_its_row_blocks(K, G, clip):
+    """A matrix of more than 2^22 words (four words per thread, a ragged tail) gives the bits of its row blocks (one word
+    per thread), and its last row the oracle's."""
+    N, Kd = 2051, 16384
+    w = torch.randn(N, Kd, generator=torch.Generator(device=DEV).manual_seed(G), device=DEV).half()
+    packed, sz = torch.empty(N, Kd // 8, dtype=torch.int32, device=DEV), torch.empty(N, Kd // G, 2, dtype=torch.half, device=DEV)
+    p2, s2 = torch.empty_like(packed), torch.empty_like(sz)
+    K.quantize_w4(w, packed, sz, G, clip)
+    for r0 in range(0, N, 1500):
+        r = slice(r0, min(N, r0 + 1500))
+        K.quantize_w4(w[r], p2[r], s2[r], G, clip)
+    assert torch.equal(packed, p2) and torch.equal(sz.view(torch.int16), s2.view(torch.int16))
+    q, s, z = Q.quantize(w[-1:].cpu().numpy(), G, clip)
+    if not clip:                                        # (with clip the oracle's fp32 error sums may break near-ties otherwise)
+        assert np.array_equal(packed[-1:].cpu().numpy(), Q.pack(q))
+
+
 def test_ops_launch_on_the_current_stream(K):
     """The handle that every op passes on is that of torch's current stream, in the main thread and in another, inside
     and outside a stream context."""
