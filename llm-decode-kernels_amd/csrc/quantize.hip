@@ -11,9 +11,9 @@
 // factor a (fp32, as torch multiplies an fp32 tensor by a Python float) mn = min * a, mx = max * a, the scale and zero
 // above, and err = sum((clamp(rint(w / scale) + zero, 0, 15) - zero) * scale - w)^2 over the group, each term in fp32
 // exactly as the reference computes it. The terms are summed in fp64, so the choice (the first factor with the
-// smallest error, the reference's strict `err < best`) is the exact argmin of the reference's fp32 terms; the
-// reference sums them in fp32, so the two can pick different factors only where two errors agree to fp32 summation
-// noise.
+// smallest error, the reference's strict `err < best`) is the argmin of the reference's fp32 terms up to fp64 rounding: the
+// eight terms of a word in order, then the words of the group pairwise, the farthest lanes first. The reference sums them
+// in fp32, so the two can pick different factors only where two errors agree to fp32 summation noise.
 //
 // One lane per packed word (8 weights, one 16-byte load), 1 or 4 words per thread (kManyWords); the G/8 lanes of a group are
 // consecutive in one wave (G <= 512) and reduce min / max (and the clip errors) by DPP within 16 lanes, by shuffles
@@ -60,21 +60,22 @@ __device__ __forceinline__ float code(float quotient, float zero) {
   return __builtin_amdgcn_fmed3f(rintf(quotient) + zero, 0.0f, 15.0f);
 }
 
-// the partner's value at lane distance O within a group (O a power of two): DPP patterns whose partner lies in the
-// block of O lanes that the XOR partner lies in (all lanes of such a block hold the same value when this is used in
-// ascending order of O)
+// the value of lane ^ O (O a power of two): DPP within 16 lanes, a shuffle beyond. Lane ^ 4 is lane ^ 7 (row_half_mirror)
+// of lane ^ 3 (quad_perm).
 template <int O>
 __device__ __forceinline__ float partner(float v) {
-  if constexpr (O == 1)
+  if constexpr (O == 1) {
     return DK_DPP_F32(v, 0xB1, 0xF);   // quad_perm [1,0,3,2]
-  else if constexpr (O == 2)
+  } else if constexpr (O == 2) {
     return DK_DPP_F32(v, 0x4E, 0xF);   // quad_perm [2,3,0,1]
-  else if constexpr (O == 4)
-    return DK_DPP_F32(v, 0x141, 0xF);  // row_half_mirror
-  else if constexpr (O == 8)
-    return DK_DPP_F32(v, 0x140, 0xF);  // row_mirror
-  else
+  } else if constexpr (O == 4) {
+    const float t = DK_DPP_F32(v, 0x1B, 0xF);  // quad_perm [3,2,1,0]
+    return DK_DPP_F32(t, 0x141, 0xF);
+  } else if constexpr (O == 8) {
+    return DK_DPP_F32(v, 0x128, 0xF);  // row_ror:8
+  } else {
     return __shfl_xor(v, O, kWave);
+  }
 }
 template <int O>
 __device__ __forceinline__ double partner(double v) {
@@ -83,19 +84,20 @@ __device__ __forceinline__ double partner(double v) {
   const float hi = partner<O>(__builtin_bit_cast(float, (uint32_t)(b >> 32)));
   return __builtin_bit_cast(double, (uint64_t)__builtin_bit_cast(uint32_t, hi) << 32 | __builtin_bit_cast(uint32_t, lo));
 }
-template <int WPG, int O = 1>
+// over the WPG lanes of a group, from the farthest partner to the nearest
+template <int WPG>
 __device__ __forceinline__ void group_range(float& lo, float& hi) {
-  if constexpr (O < WPG) {
-    lo = fminf(lo, partner<O>(lo));
-    hi = fmaxf(hi, partner<O>(hi));
-    group_range<WPG, 2 * O>(lo, hi);
+  if constexpr (WPG > 1) {
+    lo = fminf(lo, partner<WPG / 2>(lo));
+    hi = fmaxf(hi, partner<WPG / 2>(hi));
+    group_range<WPG / 2>(lo, hi);
   }
 }
-template <int WPG, int O = 1>
+template <int WPG>
 __device__ __forceinline__ void group_total(double& e) {
-  if constexpr (O < WPG) {
-    e += partner<O>(e);
-    group_total<WPG, 2 * O>(e);
+  if constexpr (WPG > 1) {
+    e += partner<WPG / 2>(e);
+    group_total<WPG / 2>(e);
   }
 }
 

@@ -169,6 +169,37 @@ def test_quantize_ties_and_tails(K, N, Kd, G, clip):
     assert np.array_equal(sz.cpu().numpy().view(np.uint16), Q.pack_scale_zero(s, z).view(np.uint16))
 
 
+@pytest.mark.parametrize("G", [128, 256, 512])
+def test_quantize_clip_sums_in_a_fixed_order(K, G):
+    """Groups whose squared errors under the factors 1.0 and 0.75 are equal in exact arithmetic (counts below, in units of
+    the scale 32), all other factors being worse, with values of 2^-24 that make the fp64 sums inexact: the choice is that
+    of the documented order (the terms of a word, then lanes pairwise from the farthest)."""
+    counts = {1.375: 67, 2.125: 8, 2.25: 1, 4.5: 22, 5.25: 2, 9.0: 2, 15.0: 1}
+    base = np.concatenate([np.full(n, 32 * t) for t, n in counts.items()])
+    rng = np.random.default_rng(G)
+    w = np.stack([rng.permutation(np.concatenate([base, rng.integers(0, 4096, G - len(base)) * 2.0 ** -24]))
+                  for _ in range(1000)]).astype(np.float16)
+
+    def total(scale, order):
+        v = w.astype(np.float32)
+        d = np.clip(np.rint(v / scale), 0, 15) * scale - v
+        t = (d * d).astype(np.float64).reshape(len(w), -1, 8)
+        e = np.zeros(t.shape[:2])
+        for i in range(8):
+            e = e + t[:, :, i]
+        for o in order:
+            e = e + e[:, np.arange(e.shape[1]) ^ o]
+        return e[:, 0]
+
+    far = [G // 8 >> i for i in range(1, (G // 8).bit_length())]
+    pick = lambda order: np.where(total(np.float32(24), order) < total(np.float32(32), order), 24.0, 32.0)
+    assert 0.1 < (pick(far) != pick(far[::-1])).mean()          # the order matters for these rows
+    packed = torch.empty(1000, G // 8, dtype=torch.int32, device=DEV)
+    sz = torch.empty(1000, 1, 2, dtype=torch.half, device=DEV)
+    K.quantize_w4(torch.from_numpy(w).to(DEV), packed, sz, G, True)
+    assert np.array_equal(sz[:, 0, 0].cpu().numpy(), pick(far).astype(np.float16))
+
+
 @pytest.mark.parametrize("G", [32, 128, 512])
 @pytest.mark.parametrize("clip", [False, True])
 def test_quantize_large_equals_its_row_blocks(K, G, clip):
