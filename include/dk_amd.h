@@ -209,10 +209,12 @@ int dk_gemm_w4a16(const void* packed, const void* sz, const void* x, void* y, in
  * epilogue 2 (shapes that split only; y unused, may be NULL): the partials alone, left in the workspace for a reader
  * that sums them (dk_rmsnorm_rows_parts), which saves the second launch; it takes the whole workspace.
  * dk_gemm_w4a16_ws_splits says what a call does: the k ranges it runs over with a workspace of that many bytes (1: it
- * does not split), 0 where it refuses. Like dk_gemm_w4a16, no counterpart in the reference.
+ * does not split), 0 where it refuses; dk_gemm_w4a16_kernel names the kernel and tile that such a call runs (a static
+ * string, "" where there is none; both are host-only). Like dk_gemm_w4a16, no counterpart in the reference.
  */
 size_t dk_gemm_w4a16_workspace_bytes(int M, int N, int K, int group, int epilogue);
 int dk_gemm_w4a16_ws_splits(int M, int N, int K, int group, int epilogue, size_t workspace_bytes);
+const char* dk_gemm_w4a16_kernel(int M, int N, int K, int group, int epilogue, int splits);
 int dk_gemm_w4a16_ws(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int group,
                      int epilogue, void* workspace, size_t workspace_bytes, void* stream);
 

@@ -282,6 +282,12 @@ int dk_gemm_w4a16_ws_splits(int M, int N, int K, int group, int epilogue, size_t
   return s;
 }
 
+const char* dk_gemm_w4a16_kernel(int M, int N, int K, int group, int epilogue, int splits) {
+  if (M <= 0 || N <= 0 || K <= 0 || group < 32 || !pow2(group) || K % 32 != 0 || K % group != 0) return "";
+  if (splits < 1 || splits > dk::gemm_w4a16_splits(M, N, K, ilog2(group), epilogue)) return "";
+  return dk::gemm_w4a16_kernel_name(M, N, K, ilog2(group), epilogue, splits);
+}
+
 int dk_gemm_w4a16_ws(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int group,
                      int epilogue, void* workspace, size_t workspace_bytes, void* stream) {
   const bool parts = epilogue == 2;  // the fp32 split partials alone, left in the workspace (y unused)

@@ -269,6 +269,15 @@ int gemm_thin_splits(int M, int N, int K, int log2G) {
   return tiles * s >= 128 && s > 1 ? s : 1;
 }
 
+const char* gemm_thin_name(int N, int splits) {
+  switch (splits > 1 ? 128 : thin_rows(N)) {
+    case 128: return "thin 128";
+    case 64: return "thin 64";
+    case 32: return "thin 32";
+    default: return "thin 16";
+  }
+}
+
 void launch_gemm_thin(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
                       int epilogue, int splits, hipStream_t st) {
   if (splits > 1) {  // y = the partials

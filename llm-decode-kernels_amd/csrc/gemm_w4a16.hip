@@ -911,20 +911,57 @@ int gemm_w4a16_tile(int M, int N, int K, int log2G) {
   return 10 * tile + kgr;
 }
 
+namespace {
+
+// What a call runs (over `splits` k ranges): the kernel of few tokens, a tiling of the register-stationary kernel, a tile
+// of the wide one, or the 16x16x16 kernel (none of them).
+struct GemmChoice {
+  bool thin;
+  RsId rs;
+  int wide;
+};
+GemmChoice choose(int M, int N, int K, int log2G, int splits) {
+  if (gemm_thin_fits(M, N, K, log2G)) return {true, kRsNone, 0};
+  double sc;
+  const RsId rs = splits > 1 ? rs_best(M, N, splits, &sc).id : rs_unsplit(M, N, K, log2G);
+  return {false, rs, rs == kRsNone ? gemm_w4a16_tile(M, N, K, log2G) : 0};
+}
+
+}  // namespace
+
+const char* gemm_w4a16_kernel_name(int M, int N, int K, int log2G, int /*epilogue*/, int splits) {
+  const GemmChoice c = choose(M, N, K, log2G, splits);
+  if (c.thin) return gemm_thin_name(N, splits);
+  switch (c.rs) {
+    case kRs512x128: return "rs 512x128 w8";
+    case kRs256x128: return "rs 256x128 w8";
+    case kRs256x64: return "rs 256x64 w8";
+    case kRs256x128w4: return "rs 256x128 w4";
+    case kRs128x128w4: return "rs 128x128 w4";
+    case kRs128x64w4: return M < 64 ? "rs 128x64 w4 few" : "rs 128x64 w4";
+    default: break;
+  }
+  switch (c.wide) {
+    case 31: return "wide 128x128";
+    case 21: return "wide 128x64";
+    case 22: return "wide 128x64 kg2";
+    case 11: return "wide 64x64";
+    case 12: return "wide 64x64 kg2";
+    case 14: return "wide 64x64 kg4";
+    default: return "16x16x16";
+  }
+}
+
 void launch_gemm_w4a16(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
                        int epilogue, int splits, void* ws, hipStream_t st) {
-  if (gemm_thin_fits(M, N, K, log2G)) {
+  const GemmChoice c = choose(M, N, K, log2G, splits);
+  if (c.thin) {
     launch_gemm_thin(packed, sz, x, splits > 1 ? ws : y, M, N, K, log2G, splits > 1 ? 2 : epilogue, splits, st);
     if (splits > 1 && epilogue != 2) launch_splitk_reduce(ws, splits, y, M, N, st);
     return;
   }
-  if (splits > 1) {
-    double sc;
-    return launch_rs_id(rs_best(M, N, splits, &sc).id, packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
-  }
-  const RsId rs = rs_unsplit(M, N, K, log2G);
-  if (rs != kRsNone) return launch_rs_id(rs, packed, sz, x, y, M, N, K, log2G, epilogue, 1, nullptr, st);
-  switch (gemm_w4a16_tile(M, N, K, log2G)) {
+  if (c.rs != kRsNone) return launch_rs_id(c.rs, packed, sz, x, y, M, N, K, log2G, epilogue, splits, ws, st);
+  switch (c.wide) {
     case 31: launch_wide<128, 128, 1>(packed, sz, x, y, M, N, K, log2G, epilogue, st); return;
     case 21: launch_wide<128, 64, 1>(packed, sz, x, y, M, N, K, log2G, epilogue, st); return;
     case 22: launch_wide<128, 64, 2>(packed, sz, x, y, M, N, K, log2G, epilogue, st); return;

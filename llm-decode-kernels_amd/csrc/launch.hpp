@@ -78,11 +78,14 @@ void launch_gemm_w4a16(const void* packed, const void* sz, const void* x, void* 
 // fewest that a workspace must hold
 int gemm_w4a16_splits(int M, int N, int K, int log2G, int epilogue);
 int gemm_w4a16_min_splits(int M, int N, int K, int log2G, int epilogue);
+// the kernel and tile of a call over that many k ranges
+const char* gemm_w4a16_kernel_name(int M, int N, int K, int log2G, int epilogue, int splits);
 
 // The GEMM of a few tokens (gemm_thin.hip): whether a shape takes it, the k ranges it splits into when a workspace is
-// given (1: it does not split), and its launch (splits > 1: y receives the fp32 partials [splits, M, N]).
+// given (1: it does not split), its tile, and its launch (splits > 1: y receives the fp32 partials [splits, M, N]).
 bool gemm_thin_fits(int M, int N, int K, int log2G);
 int gemm_thin_splits(int M, int N, int K, int log2G);
+const char* gemm_thin_name(int N, int splits);
 void launch_gemm_thin(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
                       int epilogue, int splits, hipStream_t st);
 

@@ -34,6 +34,7 @@ SIGNATURES = {
     "dk_gemm_w4a16": ([_P, _P, _P, _P, _I, _I, _I, _I, _I, _P], _I),
     "dk_gemm_w4a16_workspace_bytes": ([_I, _I, _I, _I, _I], _Z),
     "dk_gemm_w4a16_ws_splits": ([_I, _I, _I, _I, _I, _Z], _I),
+    "dk_gemm_w4a16_kernel": ([_I, _I, _I, _I, _I, _I], ctypes.c_char_p),
     "dk_gemm_w4a16_ws": ([_P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _Z, _P], _I),
     "dk_rope_append_rows": ([_P, _P, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P], _I),
     "dk_rmsnorm_rows_parts": ([_P, _P, _I, ctypes.c_longlong, _P, _P, _P, _I, _I, _F, _P], _I),
@@ -268,6 +269,10 @@ class DecodeKernels:
     def gemm_workspace_bytes(self, M, N, K, group, epilogue=0):
         """Bytes of split-K workspace dk_gemm_w4a16_ws uses for this shape (0: it does not split)."""
         return int(self.lib.dk_gemm_w4a16_workspace_bytes(int(M), int(N), int(K), int(group), int(epilogue)))
+
+    def gemm_kernel(self, M, N, K, group, epilogue=0, splits=1):
+        """Name of the kernel and tile that a GEMM of this shape runs over that many k ranges."""
+        return self.lib.dk_gemm_w4a16_kernel(int(M), int(N), int(K), int(group), int(epilogue), int(splits)).decode()
 
     def gemm_w4a16(self, packed, sz, x, y, group, epilogue=0, workspace=None):
         """y = x . dequant(W)^T (epilogue 1: SwiGLU of interleaved gate/up rows); `workspace` (a CUDA tensor of

@@ -305,6 +305,16 @@ def test_gemm_workspace_smaller_than_the_need(lib, M, N, K, S, least):
     assert lib.dk_gemm_w4a16_ws_splits(512, 4096, 4096, 128, 2, 1 << 30) == 0
 
 
+def test_gemm_kernel_names(lib):
+    name = lambda M, N, K, G, epi=0, S=1: lib.dk_gemm_w4a16_kernel(M, N, K, G, epi, S).decode()
+    assert name(16, 28672, 4096, 128, 1) == "thin 128" and name(16, 2048, 2048, 128) == "thin 16"
+    assert name(16, 4096, 14336, 128, 0, 8) == "thin 128" and name(48, 28672, 4096, 128) == "rs 128x64 w4 few"
+    assert name(512, 28672, 4096, 128, 1) == "rs 512x128 w8" and name(512, 2048, 2048, 128) == "wide 64x64 kg4"
+    assert name(512, 28672, 4096, 32) == "wide 128x128" and name(7, 100, 96, 32) == "16x16x16"
+    assert name(0, 100, 96, 32) == name(7, 100, 96, 64) == name(7, 100, 96, 32, 0, 0) == name(7, 100, 90, 32) == ""
+    assert name(7, 100, 96, 32, 0, 2) == name(512, 4096, 14336, 128, 1, 4) == ""       # more ranges than the shape has
+
+
 def test_prefill_validation(lib):
     g = lambda **kw: _err(lib, lib.dk_gemm_w4a16(*dict(dict(p=A16, sz=A16, x=A16, y=B16, M=64, N=128, K=256, G=128,
                                                             epi=0), **kw).values(), None))
