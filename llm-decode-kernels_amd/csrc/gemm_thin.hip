@@ -217,10 +217,12 @@ gemm_w4a16_thin(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int
 // Weight rows per workgroup of the unsplit kernel: the most that still give 160 workgroups, since every workgroup reads
 // all of X through its CU and the weights want every CU. us at M 16 with 128 / 64 / 32 / 16 rows: 28672 x 4096
 // 23.4 28.3 33.3 43.2; 11264 x 2048 13.5 9.0 10.3 13.4; 6144 x 4096 21.5 13.8 9.9 13.0; 4096 x 4096 20.9 13.6 9.6 7.9.
+// 16 rows up to one round of the CUs only: from 17 tokens on a workgroup's LDS fills a CU, and a few workgroups over 256
+// take a second round (N 4992, K 1280, M 18: 12.3 us with 16 rows, 6.7 with 32; at 16 tokens and less 4 to 20% less too).
 int thin_rows(int N) {
   for (int rows = 128; rows > 16; rows /= 2)
     if (N / rows >= 160) return rows;
-  return 16;
+  return N > 16 * 256 ? 32 : 16;
 }
 
 template <int TI, int MT, int RWV, int KG, int CK, int EPI>
@@ -259,10 +261,11 @@ bool gemm_thin_fits(int M, int N, int K, int log2G) {
 
 // k ranges over 128-row tiles when a workspace is given: long rows (K >= 8192) of few tiles, the fewest that make 192
 // workgroups while every K group keeps 3 chunks (4096 x 14336 at M 32, S 8: 23.2 us with the reduce launch against
-// 28.4 unsplit; 20.1 against 19.7 at M 16, where the reader that sums the partials itself saves the launch).
+// 28.4 unsplit; 20.1 against 19.7 at M 16, where the reader that sums the partials itself saves the launch). From 160
+// workgroups of 64 rows on the unsplit kernel has its CUs (12000 x 8192 at M 32: 30.0 us, split 4 ways 36.6).
 int gemm_thin_splits(int M, int N, int K, int log2G) {
   if (!gemm_thin_fits(M, N, K, log2G) || K % 256 != 0 || N % 4 != 0) return 1;
-  if (K < 8192) return 1;
+  if (K < 8192 || N / 64 >= 160) return 1;
   const int tiles = (N + 127) / 128, nk = K / 512;  // chunks per group of an unsplit workgroup
   int s = 1;
   while (s < 16 && tiles * s < 192 && nk / (2 * s) >= 3) s *= 2;

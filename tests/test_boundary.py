@@ -308,6 +308,8 @@ def test_gemm_workspace_smaller_than_the_need(lib, M, N, K, S, least):
 def test_gemm_kernel_names(lib):
     name = lambda M, N, K, G, epi=0, S=1: lib.dk_gemm_w4a16_kernel(M, N, K, G, epi, S).decode()
     assert name(16, 28672, 4096, 128, 1) == "thin 128" and name(16, 2048, 2048, 128) == "thin 16"
+    assert name(18, 4992, 1280, 128) == name(16, 5119, 2048, 64) == "thin 32" and name(18, 4096, 1280, 128) == "thin 16"
+    assert lib.dk_gemm_w4a16_workspace_bytes(32, 12000, 8192, 128, 0) == 0 and name(32, 12000, 8192, 128) == "thin 64"
     assert name(16, 4096, 14336, 128, 0, 8) == "thin 128" and name(48, 28672, 4096, 128) == "rs 128x64 w4 few"
     assert name(512, 28672, 4096, 128, 1) == "rs 512x128 w8" and name(512, 2048, 2048, 128) == "wide 64x64 kg4"
     assert name(512, 28672, 4096, 32) == "wide 128x128" and name(7, 100, 96, 32) == "16x16x16"
