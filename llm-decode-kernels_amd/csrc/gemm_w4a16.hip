@@ -796,13 +796,14 @@ RsId rs_unsplit(int M, int N, int K, int log2G) {
 
 // Split-K (a workspace given, epilogue 0 or 2 = the partials alone): the k ranges S, 1 if the shape does not split. The
 // partials cost traffic (S x M x N x 4 bytes, written and read back) and, unless the next norm sums them, a launch.
-//   * M >= 768: the S in 1, 2, 4 (16 chunks of 128 per range at least) with the best rate over its best tiling, the
+//   * M >= 768 and the unsplit kernel has its tiles: the S in 1, 2, 4 (16 chunks of 128 per range at least) with the best rate over its best tiling, the
 //     partials priced at 800 S / K of the product's time; no split unless 5% better, nor where K is under 64 chunks and
 //     the unsplit kernel has its tiles. 4096 x 14336 at M 2048 228 us unsplit (256 x 128) against 298 split 2 ways over
 //     256 x 64 tiles of four waves, at M 1024 122 split 4 ways over 512 x 128 (125 split 2 ways over 256 x 128) against 148.
-//   * below: when the unsplit kernel lacks its tiles or K has 64 chunks, the smallest power of two that gives 384
+//   * otherwise, when the unsplit kernel lacks its tiles or K has 64 chunks, the smallest power of two that gives 384
 //     workgroups of 256 x 64 (else 128 x 64) while every range keeps 16 chunks, if that reaches 192 (4096 x 14336 at M 512:
-//     S 4; TinyLlama's qkv 2560 x 2048 at S 4, 4 chunks per range: 27 us against 19 unsplit).
+//     S 4; 768 x 4096 at M 1600, 150 tiles, S 2: 25.8 us against 46.0 unsplit on the wide kernel; 256 x 16384 at M 768 20.9
+//     at S 8 against 30.7 at S 4; TinyLlama's qkv 2560 x 2048 at S 4, 4 chunks per range: 27 us against 19 unsplit).
 //   * up to 128 tokens the partials are small and the alternative is the wide kernel with a few tiles, so there shorter
 //     ranges (5 chunks) pay while the 128 x 64 tiles alone leave three quarters of the CUs idle: 4096 x 14336 at M 64 20.8 us
 //     against 66.2, 4096 x 4096 at M 33 / 64 / 128 13.0 / 13.6 / 16.3 against 18.9 / 20.5 / 19.9, 2048 x 5632 at 64
@@ -848,8 +849,8 @@ int gemm_w4a16_splits(int M, int N, int K, int log2G, int epilogue) {
   if ((epilogue == 0 || epilogue == 2) && gemm_thin_fits(M, N, K, log2G)) return gemm_thin_splits(M, N, K, log2G);
   if (!may_split(M, N, K, log2G, epilogue)) return 1;
   const int nk = K / kRsK;
-  if (M >= 768) {
-    if (nk < 64 && rs_unsplit(M, N, K, log2G) != kRsNone) return 1;
+  if (M >= 768 && rs_unsplit(M, N, K, log2G) != kRsNone) {
+    if (nk < 64) return 1;
     int best = 1;
     double top;
     rs_best(M, N, 1, &top);
