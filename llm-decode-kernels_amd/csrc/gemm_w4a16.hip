@@ -26,6 +26,8 @@
 // buffers, one barrier per chunk).
 //   Operands (lane l = 16 g + c): A = X rows, lane l holds X[row c][k 4g..4g+3]; B = W^T, lane l holds
 //   W[col c][k 4g..4g+3]; the accumulator leaves lane l with Y[rows 4g..4g+3][col c].
+#include <math.h>
+
 #include "common.hpp"
 #include "launch.hpp"
 #include "w4_common.hpp"
@@ -735,47 +737,54 @@ void launch_wide(const void* packed, const void* sz, const void* x, void* y, int
 
 
 // Tilings of the register-stationary kernel: weight rows per wave, tokens, waves per workgroup (rows x waves = the
-// tile's weight rows), and the output a CU makes in a given time when it has a full tile, relative to the first (chunk
-// time of a CU-filling grid: 512 x 128 3.5 us, 256 x 128 2.0, 256 x 64 1.2; two 256 x 128 tiles of four waves 3.9, one
-// 2.1). Eight-wave tiles share each staged X among twice the rows (with the staging taken out of the four-wave kernel,
-// 28672 x 4096 at M 512 runs in 114 us instead of 132), four-wave ones drain more smoothly over many rounds.
+// tile's weight rows). Eight-wave tiles share each staged X among twice the rows (with the staging taken out of the
+// four-wave kernel, 28672 x 4096 at M 512 runs in 114 us instead of 132), four-wave ones drain more smoothly over many
+// rounds.
+// The numbers give a launch's time in us (rs_us): with q workgroups per CU on average, L = ceil(q) on the busiest, and k
+// ranges of C chunks,
+//   fill + (tile + (ragged)) L + C (L == 1 ? c1 - k1 (1 - q) : c2 L + d2 - k2 (L - q)):
+// `tile` is a workgroup's prologue and epilogue, `ragged` what element-wise stores (N % 4 != 0; a third with the SwiGLU
+// epilogue) add to it, c1 the time of a chunk where every CU has one workgroup, c2 per workgroup where it has more (two or
+// four of the smaller tiles run side by side), and the k terms what CUs left idle give the others (power). Fitted to 13600
+// shapes of 8 to 128 chunks, N to 32768 and M 33 to 2048, each tiling timed beside the others in a random order, those
+// within 15% of the fastest weighing in: 4 to 6% off.
 enum RsId { kRsNone, kRs512x128, kRs256x128, kRs256x64, kRs256x128w4, kRs128x128w4, kRs128x64w4 };
 struct RsTiling {
   RsId id;
   int rw, bm, nw;
-  double rate;
+  double fill, tile, ragged, c1, k1, c2, d2, k2;
 };
 constexpr RsTiling kRsTilings[] = {
-    {kRs512x128, 64, 128, 8, 1.0},    {kRs256x128, 32, 128, 8, 0.875},  {kRs256x64, 32, 64, 8, 0.73},
-    {kRs256x128w4, 64, 128, 4, 0.88}, {kRs128x128w4, 32, 128, 4, 0.72}, {kRs128x64w4, 32, 64, 4, 0.64}};
+    {kRs512x128, 64, 128, 8, 3.25, 9.82, 27.62, 3.45, 2.26, 3.66, -0.42, 1.91},
+    {kRs256x128, 32, 128, 8, 3.55, 4.49, 13.97, 1.87, 1.15, 1.91, -0.12, 0.88},
+    {kRs256x64, 32, 64, 8, 2.74, 2.44, 6.40, 1.16, 0.36, 1.10, -0.03, 0.52},
+    {kRs256x128w4, 64, 128, 4, 6.39, 2.25, 13.60, 1.95, 0.71, 1.95, -0.22, 0.87},
+    {kRs128x128w4, 32, 128, 4, 4.65, 1.47, 6.63, 1.10, 0.29, 1.08, -0.12, 0.54},
+    {kRs128x64w4, 32, 64, 4, 2.64, 1.54, 2.48, 0.78, 0.09, 0.58, 0.09, 0.29}};
 constexpr int kCus = 256, kRsMinM = 33;
 
-// The tiling with the most output per time over S k ranges of an M x N output: its rate times the share of the CUs'
-// tile area that is output, rounds of 256 tiles counted whole. Measured against the tiling that the count of tiles
-// alone chose before, us: 28672 x 4096 at M 333 / 512 / 1024 101 / 117.6 / 231.6 (512 x 128) against 117 / 124 / 247
-// (256 x 128, four waves; at M 2048 that one keeps, 456 against 464); 11264 x 2048 at 333 / 512 29.8 / 32.1 (256 x 128)
-// against 34.8 / 35.7, at 1024 56.7 (512 x 128) against 62.1; 6144 x 4096 at 512 / 1024 / 2048 38.1 / 58.2 / 104.7
-// against 42.7 / 65.0 / 115; 4096 x 4096 at 2048 70.0 against 74.8; 2560 x 2048 at 1024 / 2048 20.0 / 30.5 against
-// 22.5 / 33.1; 2048 x 2048 at 2048 24.2 against 27.1.
-RsTiling rs_best(int M, int N, int S, double* score) {
-  RsTiling best = {kRsNone, 0, 0, 0, 0.0};
-  *score = 0.0;
+double rs_us(const RsTiling& t, int M, int N, int K, int S, int epilogue) {
+  const int rows = t.nw * t.rw;
+  const double q = (double)((N + rows - 1) / rows) * ((M + t.bm - 1) / t.bm) * S / kCus, L = ceil(q);
+  const double ragged = (N & 3) == 0 ? 0.0 : epilogue == 1 ? t.ragged / 3 : t.ragged;
+  const double chunk = L <= 1.0 ? t.c1 - t.k1 * (1.0 - q) : t.c2 * L + t.d2 - t.k2 * (L - q);
+  return t.fill + (t.tile + ragged) * L + (double)K / kRsK / S * chunk;
+}
+
+// The tiling of the least time over S k ranges. Against the tiling that the count of tiles alone chose before, on
+// 7800 unsplit shapes: 0.947 of its time on average, over 1.04 on one shape in 600; us: 28672 x 4096 at M
+// 333 / 512 / 1024 101 / 117.6 / 231.6 (512 x 128) against 117 / 124 / 247 (256 x 128, four waves; at M 2048 that one
+// keeps, 456 against 464); 11264 x 2048 at 333 / 512 29.8 / 32.1 (256 x 128) against 34.8 / 35.7; 6144 x 4096 at 1024 /
+// 2048 58.2 / 104.7 against 65.0 / 115; 4096 x 4096 at 2048 70.0 against 74.8; 2560 x 2048 at 1024 / 2048 20.0 / 30.5
+// against 22.5 / 33.1.
+RsId rs_best(int M, int N, int K, int S, int epilogue, double* us) {
+  RsId best = kRsNone;
   for (const RsTiling& t : kRsTilings) {
     if (N < t.nw * t.rw || (M < t.bm && !(t.id == kRs128x64w4 && M >= kRsMinM))) continue;
-    const long long tiles = (long long)((N + t.nw * t.rw - 1) / (t.nw * t.rw)) * ((M + t.bm - 1) / t.bm) * S;
-    double rounds = (double)((tiles + kCus - 1) / kCus), rate = t.rate;
-    if (t.nw == 4 && t.bm == 128 && tiles > 2 * kCus) {
-      // CUs refill one workgroup at a time (6144 x 4096 at M 1500: 128 x 128 tiles in 2.25 rounds 99 us, 512 x 128 ones
-      // in 0.56 of a round 109)
-      rounds = (double)tiles / kCus + 0.3;
-      rate *= 1.045;
-    } else if (t.id == kRs256x128w4 && tiles <= kCus) {
-      rate = 0.81;  // one workgroup per CU
-    }
-    const double sc = rate * M * N * S / (rounds * kCus * t.nw * t.rw * t.bm);
-    if (sc > *score) {
-      *score = sc;
-      best = t;
+    const double v = rs_us(t, M, N, K, S, epilogue);
+    if (best == kRsNone || v < *us) {
+      *us = v;
+      best = t.id;
     }
   }
   return best;
@@ -788,32 +797,32 @@ bool rs_takes(int M, int N, int K, int log2G) {
 }
 // unsplit from 160 tiles of 128 x 64 on; below, the wide kernel's 64 x 64 tiles reach more CUs (TinyLlama o and down at
 // M 512: 11.4 and 31.3 us against 13.8 and 34.2 at 128 tiles)
-RsId rs_unsplit(int M, int N, int K, int log2G) {
-  if (!rs_takes(M, N, K, log2G) || (long long)((N + 127) / 128) * ((M + 63) / 64) < 160) return kRsNone;
-  double sc;
-  return rs_best(M, N, 1, &sc).id;
+bool rs_fills(int M, int N, int K, int log2G) {
+  return rs_takes(M, N, K, log2G) && (long long)((N + 127) / 128) * ((M + 63) / 64) >= 160;
 }
 
 // Split-K (a workspace given, epilogue 0 or 2 = the partials alone): the k ranges S, 1 if the shape does not split. The
 // partials cost traffic (S x M x N x 4 bytes, written and read back) and, unless the next norm sums them, a launch.
-//   * M >= 768 and the unsplit kernel has its tiles: the S in 1, 2, 4 (16 chunks of 128 per range at least) with the best rate over its best tiling, the
-//     partials priced at 800 S / K of the product's time; no split unless 5% better, nor where K is under 64 chunks and
-//     the unsplit kernel has its tiles. 4096 x 14336 at M 2048 228 us unsplit (256 x 128) against 298 split 2 ways over
+//   * M >= 768 and the unsplit kernel has its tiles: the S in 1, 2, 4 (16 chunks of 128 per range at least) of the least time
+//     over its best tiling, the partials priced at half of what a reduce launch reads them in (7 TB/s: most readers are
+//     norms that read them anyway); no split unless 5% better, nor where K is under 64 chunks. 4096 x 14336 at M 2048 228 us unsplit (256 x 128) against 298 split 2 ways over
 //     256 x 64 tiles of four waves, at M 1024 122 split 4 ways over 512 x 128 (125 split 2 ways over 256 x 128) against 148.
 //   * otherwise, when the unsplit kernel lacks its tiles or K has 64 chunks, the smallest power of two that gives 384
 //     workgroups of 256 x 64 (else 128 x 64) while every range keeps 16 chunks, if that reaches 192 (4096 x 14336 at M 512:
 //     S 4; 768 x 4096 at M 1600, 150 tiles, S 2: 25.8 us against 46.0 unsplit on the wide kernel; 256 x 16384 at M 768 20.9
-//     at S 8 against 30.7 at S 4; TinyLlama's qkv 2560 x 2048 at S 4, 4 chunks per range: 27 us against 19 unsplit).
+//     at S 8 against 30.7 at S 4; from M 768 on as many of 4 ranges as keep 16 chunks where even that does not reach 192:
+//     768 x 4096 at M 900 S 2 19.2 against 24.3 unsplit, 304 x 13312 at M 884 S 4 27.7 against 67.2; TinyLlama's qkv 2560 x 2048 at S 4, 4 chunks per range: 27 us against 19 unsplit).
 //   * up to 128 tokens the partials are small and the alternative is the wide kernel with a few tiles, so there shorter
 //     ranges (5 chunks) pay while the 128 x 64 tiles alone leave three quarters of the CUs idle: 4096 x 14336 at M 64 20.8 us
 //     against 66.2, 4096 x 4096 at M 33 / 64 / 128 13.0 / 13.6 / 16.3 against 18.9 / 20.5 / 19.9, 2048 x 5632 at 64
 //     12.0 against 26.4; with 96 tiles (6144 x 4096 at M 128) they lose, 21 against 19.2.
 constexpr int kSplitMinChunks = 16;
+constexpr double kPartsUs = 0.5 * 4e-6 / 7.0;  // per partial value
 
 // the second rule, without a bound on M: 1 if it does not split
 int base_splits(int M, int N, int K, int log2G, int max_rows) {
   const int nk = K / kRsK;
-  if (nk < 64 && rs_unsplit(M, N, K, log2G) != kRsNone) return 1;
+  if (nk < 64 && rs_fills(M, N, K, log2G)) return 1;
   const long long tm = (M + 63) / 64;
   for (int rows = max_rows; rows >= 128; rows /= 2) {
     const long long tiles = (N + rows - 1) / rows * tm;
@@ -849,25 +858,25 @@ int gemm_w4a16_splits(int M, int N, int K, int log2G, int epilogue) {
   if ((epilogue == 0 || epilogue == 2) && gemm_thin_fits(M, N, K, log2G)) return gemm_thin_splits(M, N, K, log2G);
   if (!may_split(M, N, K, log2G, epilogue)) return 1;
   const int nk = K / kRsK;
-  if (M >= 768 && rs_unsplit(M, N, K, log2G) != kRsNone) {
+  if (M >= 768 && rs_fills(M, N, K, log2G)) {
     if (nk < 64) return 1;
     int best = 1;
-    double top;
-    rs_best(M, N, 1, &top);
-    top *= 1.05;
+    double least, us;
+    rs_best(M, N, K, 1, 0, &least);
+    least *= 0.95;
     for (int s = 2; s <= 4 && nk / s >= kSplitMinChunks; s *= 2) {
-      double sc;
-      rs_best(M, N, s, &sc);
-      sc /= 1.0 + 800.0 * s / K;
-      if (sc > top) {
-        top = sc;
+      rs_best(M, N, K, s, 0, &us);
+      us += s * kPartsUs * M * N;
+      if (us < least) {
+        least = us;
         best = s;
       }
     }
     return best;
   }
   const int base = base_splits(M, N, K, log2G, M < 64 ? 128 : 256);
-  if (base > 1 || (nk < 64 && rs_unsplit(M, N, K, log2G) != kRsNone)) return base;
+  if (base > 1 || (nk < 64 && rs_fills(M, N, K, log2G))) return base;
+  if (M >= 768) return nk >= 4 * kSplitMinChunks ? 4 : nk >= 2 * kSplitMinChunks ? 2 : 1;
   if (M <= 128) {
     const long long tiles = (long long)((N + 127) / 128) * ((M + 63) / 64);
     int s = 2;
@@ -921,17 +930,17 @@ struct GemmChoice {
   RsId rs;
   int wide;
 };
-GemmChoice choose(int M, int N, int K, int log2G, int splits) {
+GemmChoice choose(int M, int N, int K, int log2G, int epilogue, int splits) {
   if (gemm_thin_fits(M, N, K, log2G)) return {true, kRsNone, 0};
-  double sc;
-  const RsId rs = splits > 1 ? rs_best(M, N, splits, &sc).id : rs_unsplit(M, N, K, log2G);
-  return {false, rs, rs == kRsNone ? gemm_w4a16_tile(M, N, K, log2G) : 0};
+  double us;
+  if (splits > 1 || rs_fills(M, N, K, log2G)) return {false, rs_best(M, N, K, splits, epilogue, &us), 0};
+  return {false, kRsNone, gemm_w4a16_tile(M, N, K, log2G)};
 }
 
 }  // namespace
 
-const char* gemm_w4a16_kernel_name(int M, int N, int K, int log2G, int /*epilogue*/, int splits) {
-  const GemmChoice c = choose(M, N, K, log2G, splits);
+const char* gemm_w4a16_kernel_name(int M, int N, int K, int log2G, int epilogue, int splits) {
+  const GemmChoice c = choose(M, N, K, log2G, epilogue, splits);
   if (c.thin) return gemm_thin_name(N, splits);
   switch (c.rs) {
     case kRs512x128: return "rs 512x128 w8";
@@ -955,7 +964,7 @@ const char* gemm_w4a16_kernel_name(int M, int N, int K, int log2G, int /*epilogu
 
 void launch_gemm_w4a16(const void* packed, const void* sz, const void* x, void* y, int M, int N, int K, int log2G,
                        int epilogue, int splits, void* ws, hipStream_t st) {
-  const GemmChoice c = choose(M, N, K, log2G, splits);
+  const GemmChoice c = choose(M, N, K, log2G, epilogue, splits);
   if (c.thin) {
     launch_gemm_thin(packed, sz, x, splits > 1 ? ws : y, M, N, K, log2G, splits > 1 ? 2 : epilogue, splits, st);
     if (splits > 1 && epilogue != 2) launch_splitk_reduce(ws, splits, y, M, N, st);

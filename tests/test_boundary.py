@@ -286,7 +286,7 @@ def test_small_op_validation(lib):
 
 @pytest.mark.parametrize("M,N,K,S,least", [
     (16, 4096, 14336, 8, 1), (33, 4096, 4096, 4, 1), (64, 4096, 4096, 4, 1), (128, 2048, 5632, 8, 1),   # up to 128 tokens
-    (1600, 768, 4096, 2, 2), (768, 256, 16384, 8, 8), (2048, 256, 16384, 8, 8),
+    (900, 768, 4096, 2, 1), (884, 304, 13312, 4, 1), (1600, 768, 4096, 2, 2), (768, 256, 16384, 8, 8), (2048, 256, 16384, 8, 8),
     (512, 4096, 14336, 4, 4), (512, 2048, 5632, 2, 2), (767, 4096, 14336, 2, 2),                        # idle CUs, long k
     (1000, 4096, 14336, 4, 2)])
 def test_gemm_workspace_smaller_than_the_need(lib, M, N, K, S, least):
