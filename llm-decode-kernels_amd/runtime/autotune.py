@@ -251,7 +251,7 @@ def write_table(out, path):
 
 # ------------------------------------------------------------------------------------------ attention policy
 ATTN_MODELS = {64: "TINYLLAMA", 128: "LLAMA3_8B"}   # head_dim -> the model whose decode step the policy is tuned in
-ATTN_CONTEXTS = (512, 1024, 2048, 4096, 16384)
+ATTN_CONTEXTS = (512, 1024, 2048, 4096, 8192, 16384)
 ATTN_PATH = PKG / "configs" / "attn_policy.json"
 
 
@@ -271,13 +271,38 @@ def step_time_us(model, ctx, steps=24, warmup=8):
     return a.elapsed_time(b) * 1e3 / steps
 
 
+def merge_policy(entries, tuned):
+    """Policy entries by context, those of `tuned` in the place of earlier ones, and after them an open-ended copy of the
+    last (the reference's schema ends on one; the runtime's lookup takes the entries with a context of their own)."""
+    by_ctx = {e["max_ctx"]: e for e in entries if e["max_ctx"] < 1 << 30}
+    by_ctx.update({e["max_ctx"]: e for e in tuned})
+    ents = [by_ctx[c] for c in sorted(by_ctx)]
+    return ents + [dict(ents[-1], max_ctx=1 << 30)]
+
+
+SAME_STEP = 1.005   # two passes of the tuner differ by 0.2 to 0.4%
+
+
+def choose_split(times, smaller):
+    """(impl, part_size) of the least step time; the choice of the largest context among the entries `smaller` where it
+    is no slower than that within a pass's spread (a model prepared for a long context mostly runs at shorter ones)."""
+    best = min(times, key=times.get)
+    if smaller:
+        e = max(smaller, key=lambda e: e["max_ctx"])
+        kept = (e["impl"], e["part_size"])
+        if times.get(kept, float("inf")) <= SAME_STEP * times[best]:
+            return kept
+    return best
+
+
 def tune_attention(dims=(64, 128), contexts=ATTN_CONTEXTS, path=ATTN_PATH, log=print):
     """Writes configs/attn_policy.json: per head dim, entries {max_ctx, part_size, impl} (the reference's schema,
-    runtime/model.py:160-178, plus the kernel choice), the last one open-ended. Every candidate (impl 1 block kernel,
+    runtime/model.py:160-178, plus the kernel choice), the last one open-ended; entries and grid records of contexts that
+    are not tuned now stay. Every candidate (impl 1 block kernel,
     2 MFMA kernel or 3 lean MFMA kernel, split size) is timed inside the decode step of the model that has this head
     dim (graph replay at context ctx): an attention kernel costs more inside the step, interleaved with the GEMVs,
     than back to back, and by different amounts per kernel, so isolated launches would choose wrongly. The three
-    fastest candidates of each context are timed twice more, interleaved, and keep their best time."""
+    fastest candidates of each context are timed twice more, interleaved, and keep their best time (choose_split)."""
     from . import synth
     from .model import DecodeConfig, Model
     old = json.load(open(path)) if pathlib.Path(path).exists() else {}
@@ -287,7 +312,9 @@ def tune_attention(dims=(64, 128), contexts=ATTN_CONTEXTS, path=ATTN_PATH, log=p
                    "<= the prepared cap; chosen by the decode step time of the TinyLlama (head_dim 64) and Llama-3-8B "
                    "(head_dim 128) shapes on MI355X (runtime.autotune.tune_attention). 'policy' is head_dim 64, "
                    "'policy_d128' head_dim 128."}
-    grid = []
+    key = lambda D: "policy" if D == 64 else f"policy_d{D}"
+    out.update({key(D): old[key(D)] for D in sorted(ATTN_MODELS) if key(D) in old})
+    grid = [r for r in old.get("grid", []) if r["D"] not in dims or r["ctx"] not in contexts]
     for D in dims:
         shape = getattr(synth, ATTN_MODELS[D])
         cap_max = max(contexts) + 64
@@ -312,15 +339,14 @@ def tune_attention(dims=(64, 128), contexts=ATTN_CONTEXTS, path=ATTN_PATH, log=p
                     times[(impl, ps)] = min(times[(impl, ps)], step_time_us(model, ctx))
             for (impl, ps), us in times.items():
                 grid.append({"D": D, "ctx": ctx, "impl": impl, "part_size": ps, "step_us": round(us, 2)})
-            impl, ps = min(times, key=times.get)
+            impl, ps = choose_split(times, [e for e in old.get(key(D), []) + ents if e["max_ctx"] < ctx])
             best = (times[(impl, ps)], impl, ps)
             log(f"  attention D{D} ctx {ctx}: best impl {best[1]} part_size {best[2]} ({best[0]:.1f} us per step)")
             ents.append({"max_ctx": ctx, "part_size": best[2], "impl": best[1]})
-        ents[-1] = dict(ents[-1], max_ctx=1 << 30)
-        out["policy" if D == 64 else f"policy_d{D}"] = ents
+        out[key(D)] = merge_policy(old.get(key(D), []), ents)
         del model
         torch.cuda.empty_cache()
-    out["grid"] = grid
+    out["grid"] = sorted(grid, key=lambda r: (r["D"], r["ctx"]))
     write_table(out, path)
     return out
 
@@ -409,11 +435,13 @@ def main(argv=None):
     ap.add_argument("--reps", type=int, default=5)
     ap.add_argument("--out", default=None)
     ap.add_argument("--attention", action="store_true", help="tune the attention policy instead of the GEMVs")
+    ap.add_argument("--contexts", default=None, help="with --attention: the contexts to tune (default: all)")
     ap.add_argument("--step", action="store_true", help="tune the decode step's GEMV launches inside the step")
     a = ap.parse_args(argv)
     log = lambda *s: print(*s, flush=True)
     if a.attention:
-        tune_attention(path=a.out or ATTN_PATH, log=log)
+        ctxs = tuple(int(c) for c in a.contexts.split(",")) if a.contexts else ATTN_CONTEXTS
+        tune_attention(contexts=ctxs, path=a.out or ATTN_PATH, log=log)
         return
     if a.step:
         tune_step(path=a.out or CONFIG, log=log)

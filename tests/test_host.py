@@ -70,6 +70,29 @@ def test_attention_policy_entries_are_launchable():
             assert Model._policy_entry_of(pol, D, e["max_ctx"]) == e
 
 
+def test_attention_policy_is_what_the_tuner_measured():
+    """The committed entries are what the tuner chooses from the committed measurements, at every context that it visits,
+    the open-ended one a copy of the last; and a tuning pass over some contexts keeps the others' entries."""
+    import json
+    from runtime.autotune import ATTN_CONTEXTS, choose_split, merge_policy
+    from runtime.model import DecodeConfig, Model
+    pol = json.load(open(DecodeConfig().attn_policy_path))
+    for key, D in (("policy", 64), ("policy_d128", 128)):
+        assert [e["max_ctx"] for e in pol[key][:-1]] == list(ATTN_CONTEXTS)
+        for i, e in enumerate(pol[key][:-1]):
+            times = {(r["impl"], r["part_size"]): r["step_us"] for r in pol["grid"] if (r["D"], r["ctx"]) == (D, e["max_ctx"])}
+            assert choose_split(times, pol[key][:i]) == (e["impl"], e["part_size"]), (D, e)
+        assert {**pol[key][-1], "max_ctx": 0} == {**pol[key][-2], "max_ctx": 0}
+    assert choose_split({(3, 80): 100.4, (3, 160): 100.0}, []) == (3, 160)
+    assert choose_split({(3, 80): 100.4, (3, 160): 100.0}, [{"max_ctx": 4096, "part_size": 80, "impl": 3}]) == (3, 80)
+    assert choose_split({(3, 80): 101.0, (3, 160): 100.0}, [{"max_ctx": 4096, "part_size": 80, "impl": 3}]) == (3, 160)
+    a, b, c = ({"max_ctx": n, "part_size": p, "impl": 3} for n, p in ((512, 96), (8192, 128), (16384, 192)))
+    assert merge_policy([], [a, b]) == [a, b, dict(b, max_ctx=1 << 30)]
+    assert merge_policy(merge_policy([], [a, b]), [c]) == [a, b, c, dict(c, max_ctx=1 << 30)]
+    assert merge_policy([a, b], [dict(b, part_size=80)])[1]["part_size"] == 80
+    assert Model._policy_entry_of({"policy": merge_policy([], [a, c])}, 64, 40000) == c
+
+
 def test_rope_theta_from_hf_configs():
     """The RoPE base comes from the config whichever way transformers stores it: the rope_theta attribute (4.x) or
     the rope_parameters dict (5.x, which has no attribute: reading only the attribute, as the reference's
