@@ -110,14 +110,32 @@ def default_gemv_config(N, K):
 TUNED_GROUP = 128
 
 
-def for_group(table, group):
+GROUP_TABLES = ("best", "best_norm", "best_gate_up", "best_step", "us", "us_norm")
+
+
+def for_group(table, group, tuned=()):
     """A tuning table ("...NxK_G128" -> entry) with entries for `group` too: a shape that was not tuned at this group size
     takes its entry of G 128. The row tiles follow N, K and the launch, hardly the group, and the defaults are far worse:
     a decode step of 8 Llama-3-8B layers at context 1000 takes 326 us instead of 377 at G 64, 340 instead of 385 at G 32,
-    315 instead of 373 at G 256 (318 at G 128); 12 TinyLlama layers 283 instead of 297 at G 64."""
+    315 instead of 373 at G 256 (318 at G 128); 12 TinyLlama layers 283 instead of 297 at G 64. `tuned`: shapes that
+    borrow nothing."""
     suffix = f"_G{TUNED_GROUP}"
-    borrowed = {k[: -len(suffix)] + f"_G{group}": v for k, v in table.items() if k.endswith(suffix)}
+    borrowed = {k[: -len(suffix)] + f"_G{group}": v for k, v in table.items()
+                if k.endswith(suffix) and _shape_of(k) not in tuned}
     return {**borrowed, **table}
+
+
+def _shape_of(key):
+    """"kind:NxK_G128" or "NxK_G128" -> "NxK"."""
+    return key.split(":")[-1].rsplit("_G", 1)[0]
+
+
+def group_tables(tab, group):
+    """The tuning tables of GROUP_TABLES for `group`. A shape with an entry of its own at this group size in any of them
+    borrows in none: a borrowed in-step choice would go ahead of its own isolated one, and a borrowed time be compared
+    with its own."""
+    tuned = {_shape_of(k) for t in GROUP_TABLES for k in tab.get(t, {}) if k.endswith(f"_G{group}")}
+    return {t: for_group(tab.get(t, {}), group, tuned) for t in GROUP_TABLES}
 
 
 class Linear:
@@ -234,14 +252,14 @@ class Model:
         self.step_cfg_override = {}
         if cfg.gemv_stage is None and Path(cfg.autotune_path).exists():
             tab = json.load(open(cfg.autotune_path))
-            t = lambda key: for_group(tab.get(key, {}), cfg.group)
-            self.gemv_table, self.gemv_norm_table = t("best"), t("best_norm")
-            self.gemv_us, self.gemv_norm_us = t("us"), t("us_norm")
-            self.gemv_gate_up_table = t("best_gate_up")
+            t = group_tables(tab, cfg.group)
+            self.gemv_table, self.gemv_norm_table = t["best"], t["best_norm"]
+            self.gemv_us, self.gemv_norm_us = t["us"], t["us_norm"]
+            self.gemv_gate_up_table = t["best_gate_up"]
             self.gemv_f16_table = tab.get("best_f16", {})
             self.gemv_f16_norm_table = tab.get("best_f16_norm", {})
             # configurations chosen by the decode step time (runtime.autotune.tune_step), ahead of the isolated tables
-            self.step_cfg_override = {k: tuple(v) for k, v in t("best_step").items()}
+            self.step_cfg_override = {k: tuple(v) for k, v in t["best_step"].items()}
 
         # paged KV cache [L, 2, pages, n_kv, P, D]; one block table shared by all layers (one sequence)
         self.n_pages = (cfg.max_ctx + cfg.page - 1) // cfg.page + 1

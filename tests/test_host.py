@@ -123,3 +123,19 @@ def test_untuned_group_borrows_the_entries_of_g128():
     assert for_group(tab, 128) == tab
     assert for_group(tab, 64) == {**tab, "rope:6144x4096_G64": [4, 4, 4, 2]}
     assert for_group(tab, 32)["2048x2048_G32"] == [4, 2, 0, 1] and for_group({}, 64) == {}
+
+
+def test_a_shape_tuned_at_its_group_borrows_nothing():
+    """A shape with an own-group entry in one table takes nothing of G 128 from the others (an in-step choice goes ahead of
+    an isolated one, and fused and plain times are compared with each other); other shapes borrow as before, and G 128
+    itself is as written."""
+    from runtime.model import GROUP_TABLES, group_tables
+    tab = {"best": {"2048x2048_G128": [4, 2, 0, 1], "2048x2048_G64": [3, 2, 1, 0], "6144x4096_G128": [4, 1, 0, 0]},
+           "best_step": {"plain:2048x2048_G128": [4, 8, 0, 0], "rope:6144x4096_G128": [4, 4, 4, 2]},
+           "us": {"2048x2048_G64": 3.0, "2048x2048_G128": 2.5}, "us_norm": {"2048x2048_G128": 2.7, "6144x4096_G128": 9.0}}
+    t = group_tables(tab, 64)
+    assert t["best"]["2048x2048_G64"] == [3, 2, 1, 0] and t["us"]["2048x2048_G64"] == 3.0
+    assert "plain:2048x2048_G64" not in t["best_step"] and "2048x2048_G64" not in t["us_norm"]
+    assert t["best_step"]["rope:6144x4096_G64"] == [4, 4, 4, 2] and t["us_norm"]["6144x4096_G64"] == 9.0
+    assert t["best"]["6144x4096_G64"] == [4, 1, 0, 0] and t["best_norm"] == {}
+    assert group_tables(tab, 128) == {k: tab.get(k, {}) for k in GROUP_TABLES}
