@@ -127,8 +127,9 @@ attn_prefill_kernel(const f16* __restrict__ qkv, const int32_t* __restrict__ pos
   }
 
   // Thread's share of a round: chunk tid % CH of token rows tid / CH + RPI i. The rows' pages are looked up a round
-  // ahead of their K / V loads (branch-free: a lookup behind a branch waits for every load in flight). Tokens past ctx
-  // or without a page read page 0's row (every cache has one) and are zeroed on the way to LDS.
+  // ahead of their K / V loads (branch-free: a lookup behind a branch waits for every load in flight). Tokens without a
+  // page read page 0's row (every cache has one), those past ctx a row of the last page (UP) or of page 0; both are zeroed
+  // on the way to LDS.
   // UP (pages of at least the 64 / CH rows that one load instruction of a wave covers): the instruction's rows lie in
   // one page, so lane i looks up the page of load i, and the load's base is computed on the scalar unit; with a page
   // per lane the address arithmetic alone took a tenth of the kernel's time.
@@ -300,7 +301,7 @@ attn_prefill_kernel(const f16* __restrict__ qkv, const int32_t* __restrict__ pos
     stage(0);
     __syncthreads();
     for (int rnd = 0; rnd < nrnd; ++rnd) {
-      fetch(rnd + 1);  // past the end: nothing is in the context, page 0's rows are read and never computed on
+      fetch(rnd + 1);  // past the end: nothing is in the context, the rows read are never computed on
       pf_fence();
       lookup(rnd + 2);
       pf_fence();
@@ -402,7 +403,8 @@ attn_prefill_kernel(const f16* __restrict__ qkv, const int32_t* __restrict__ pos
 // whether or not anything is read from LDS, 1.63 PFLOP/s at the clock that they hold; the softmax adds 40, the staging
 // of K / V 57 at four waves per workgroup and 30 at eight. Interleaving one tile's softmax with the next one's scores
 // in a wave (255 us) and two wave groups taking turns on the matrix cores behind barriers (217-225) were no faster.
-// Pages too small for one base per load instruction (UP) take the general lookup in two of the shapes.
+// Pages too small for one base per load instruction (UP) take the general lookup in two of the shapes. At D 128 the
+// (2,4,32) shape holds 256 VGPRs and spills 8, with and without UP.
 template <int D>
 void launch_prefill(const void* qkv, const int32_t* pos, const int32_t* bt, int n_bt, const void* kc, const void* vc,
                     int n_pages, int log2P, int n_q, int n_kv, int M, int max_ctx, void* out, hipStream_t st) {
@@ -423,18 +425,26 @@ void launch_prefill(const void* qkv, const int32_t* pos, const int32_t* bt, int 
       go(attn_prefill_kernel<D, 4, 1, 64, false>, 4, 256);
     else
       go(attn_prefill_kernel<D, 2, 4, 32, false>, 2, 512);
-  } else if (waves <= (D == 64 ? 512 : 256)) {
-    go(attn_prefill_kernel<D, 1, 4, 32, true>, 1, 256);
-  } else if (D == 64 && waves <= 1536) {
-    go(attn_prefill_kernel<D, 2, 2, 64, true>, 2, 256);
-  } else if (D == 128 && waves <= 640) {
-    go(attn_prefill_kernel<D, 2, 4, 32, true>, 2, 512);
-  } else if (D == 128 && waves <= 1536) {
-    go(attn_prefill_kernel<D, 4, 2, 64, true>, 4, 512);
-  } else if (D == 128 && waves >= 4096) {
-    go(attn_prefill_kernel<D, 8, 1, 64, true>, 8, 512);
+    return;
+  }
+  if constexpr (D == 64) {
+    if (waves <= 512)
+      go(attn_prefill_kernel<64, 1, 4, 32, true>, 1, 256);
+    else if (waves <= 1536)
+      go(attn_prefill_kernel<64, 2, 2, 64, true>, 2, 256);
+    else
+      go(attn_prefill_kernel<64, 4, 1, 64, true>, 4, 256);
   } else {
-    go(attn_prefill_kernel<D, 4, 1, 64, true>, 4, 256);
+    if (waves <= 256)
+      go(attn_prefill_kernel<128, 1, 4, 32, true>, 1, 256);
+    else if (waves <= 640)
+      go(attn_prefill_kernel<128, 2, 4, 32, true>, 2, 512);
+    else if (waves <= 1536)
+      go(attn_prefill_kernel<128, 4, 2, 64, true>, 4, 512);
+    else if (waves < 4096)
+      go(attn_prefill_kernel<128, 4, 1, 64, true>, 4, 256);
+    else
+      go(attn_prefill_kernel<128, 8, 1, 64, true>, 8, 512);
   }
 }
 
