@@ -318,6 +318,22 @@ def test_gemm_kernel_names(lib):
     assert name(7, 100, 96, 32, 0, 2) == name(512, 4096, 14336, 128, 1, 4) == ""       # more ranges than the shape has
 
 
+def test_gemm_tiling_cases_take_their_kernels(lib):
+    """The cases that the GPU tests of the GEMM tilings run still reach the kernels that they are there for, and leave no
+    tiling out: a rule that is tuned anew has to bring cases of its own."""
+    from helpers import GEMM_TILING_CASES
+    for kernel, M, N, K, epi, S in GEMM_TILING_CASES:
+        assert lib.dk_gemm_w4a16_kernel(M, N, K, 128, epi, S).decode() == kernel, (kernel, M, N, K, epi, S)
+        assert lib.dk_gemm_w4a16_workspace_bytes(M, N, K, 128, epi) == (S * M * N * 4 if S > 1 else 0), (kernel, M, N, K)
+    for kernel in {c[0] for c in GEMM_TILING_CASES if c[0].startswith("rs")}:
+        mine = [c for c in GEMM_TILING_CASES if c[0] == kernel]
+        unsplit = [c for c in mine if c[5] == 1]
+        assert any(c[5] > 1 for c in mine) and {c[4] for c in unsplit} == {0, 1}, kernel
+        assert {c[3] // 128 % 2 for c in unsplit} == {0, 1} and all(c[3] >= 384 for c in unsplit), kernel
+        assert any(c[2] % 16 == 0 for c in unsplit) and any(c[2] % 4 for c in unsplit), kernel
+    assert len({c[0] for c in GEMM_TILING_CASES if c[0].startswith("rs")}) == 7
+
+
 def test_prefill_validation(lib):
     g = lambda **kw: _err(lib, lib.dk_gemm_w4a16(*dict(dict(p=A16, sz=A16, x=A16, y=B16, M=64, N=128, K=256, G=128,
                                                             epi=0), **kw).values(), None))

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import DEV, assert_close, dequant_from_gpu, gen, make_cache
+from helpers import DEV, GEMM_TILING_CASES, assert_close, dequant_from_gpu, gen, make_cache
 from oracle import quant_ref as Q
 from oracle import ref_ops as R
 
@@ -29,13 +29,11 @@ def _weights(K, N, Kd, G, seed):
     return packed, sz
 
 
-# kernel coverage: K % 128 == 0 and G >= 64 -> the register-stationary kernel when a tiling has enough tiles:
-# 256 weight rows x 128 tokens (the last four cases: G 64, 128 and 256, ragged M and N, an odd chunk count),
-# 128 x 128 ((512, 11264), ragged (300, 20000), (260, 19998) with N % 4 != 0 and 3 chunks), 128 x 64 ((512, 2560),
-# ragged (130, 10002), (200, 12302) at G 64); otherwise K % 64 == 0 -> the wide kernel, tiles
-# 128 x 128, 128 x 64, 64 x 64 and 1, 2 or 4 K groups by grid size (G 32 keeps (512, 4096, 1024) on 128 x 64 with 2
-# groups and (200, 4100, 512) on 64 x 64 with 2); K % 64 == 32 -> the 16x16x16 kernel; N % 4 != 0 -> the element-wise
-# epilogue stores
+# kernel coverage (the tilings of the register-stationary kernel one by one: GEMM_TILING_CASES): K % 128 == 0 and G >= 64
+# -> the register-stationary kernel when 128 x 64 tiles make 160 workgroups, G 64, 128 and 256, ragged M and N, odd and even
+# chunk counts; otherwise K % 64 == 0 -> the wide kernel, tiles 128 x 128, 128 x 64, 64 x 64 and 1, 2 or 4 K groups by grid
+# size (G 32 keeps (512, 4096, 1024) on 128 x 64 with 2 groups and (200, 4100, 512) on 64 x 64 with 2); (7, 2560) the
+# few-token kernel; K % 64 == 32 -> the 16x16x16 kernel; N % 4 != 0 -> the element-wise epilogue stores
 @pytest.mark.parametrize("M,N,Kd,G", [(1, 64, 256, 128), (7, 2560, 2048, 128), (64, 2048, 2048, 64),
                                       (100, 1000, 5632, 128), (512, 11264, 2048, 128), (33, 4096, 4096, 32),
                                       (512, 4096, 1024, 128), (70, 999, 256, 128), (40, 300, 320, 64),
@@ -68,9 +66,8 @@ def _grid_weights(N, Kd, G, seed):
     return packed, sz, torch.from_numpy(Q.dequantize(q, scale, zero, G))
 
 
-# one case per kernel and tiling: the K % 64 == 32 kernel; the wide kernel at 64 x 64 with 1, 2 and 4 K groups,
-# 128 x 64 with 1 and 2, 128 x 128; the register-stationary tilings 256 x 128, 128 x 128, 128 x 64; split-K over
-# 256-row tiles (the 256 x 64 tiling runs split only) and over 128-row tiles
+# one case per kernel: the K % 64 == 32 kernel; the wide kernel at 64 x 64 with 1, 2 and 4 K groups, 128 x 64 with 1 and 2,
+# 128 x 128; the register-stationary one at 2 to 5 chunks and G 64, unsplit and split (its tilings: GEMM_TILING_CASES)
 @pytest.mark.parametrize("M,N,Kd,G,ws", [(20, 100, 96, 32, False), (40, 300, 320, 64, False),
                                          (200, 4100, 512, 32, False), (64, 2048, 2048, 64, False),
                                          (400, 8000, 256, 32, False), (512, 4096, 1024, 32, False),
@@ -92,9 +89,9 @@ def test_gemm_exact_on_integer_grid(K, M, N, Kd, G, ws):
     assert torch.equal(y.cpu(), want)
 
 
-# split-K (a workspace; K long or no unsplit register-stationary tiling; at least 16 k chunks per split): S = 4 over
-# 256-row tiles at Llama-3 down, S = 2 over 128-row tiles at TinyLlama down (44 chunks), S = 4 with uneven chunk
-# ranges (109 chunks) and ragged M and N, S = 4 at G 256 with M = 100 (its second token tile shifted inward)
+# split-K (a workspace; K long or no unsplit register-stationary tiling; at least 16 k chunks per split): S = 4 at Llama-3
+# down, S = 2 at TinyLlama down (44 chunks), S = 4 with uneven chunk ranges (109 chunks) and ragged M and N, S = 4 at G 256
+# with M = 100 (its second token tile shifted inward)
 @pytest.mark.parametrize("M,N,Kd,G,S", [(512, 4096, 14336, 128, 4), (512, 2048, 5632, 128, 2),
                                         (300, 4100, 13952, 64, 4), (100, 14000, 8192, 256, 4)])
 def test_gemm_splitk_matches_oracle(K, M, N, Kd, G, S):
@@ -116,7 +113,7 @@ def test_gemm_splitk_matches_oracle(K, M, N, Kd, G, S):
 
 
 # the split partials read by the next residual + RMSNorm instead of the GEMM's reduce launch: S 2 (TinyLlama down),
-# S 4 over 32-row tiles with a ragged M, S 8 (two batches of four splits in the norm's loads)
+# S 4 with a ragged M, S 8 (two batches of four splits in the norm's loads)
 @pytest.mark.parametrize("M,N,Kd,S", [(512, 2048, 5632, 2), (100, 4096, 14336, 4), (256, 1536, 16384, 8)])
 def test_rmsnorm_rows_parts_matches_reduce_then_norm(K, M, N, Kd, S):
     """gemm_w4a16_parts leaves S fp32 partials whose split-order sum, rounded once, is the reduced output, and
@@ -233,8 +230,39 @@ def test_gemm_few_tokens_exact_on_integer_grid(K, M, N, Kd, G, S):
         assert_close(act, R.swiglu_ref(torch.cat([want[:, 0::2], want[:, 1::2]], 1)), 1e-3, "swiglu of the exact rows")
 
 
-# the register-stationary tilings with ragged M and N: 512 x 128, 256 x 128 and 256 x 64 in eight waves, 256 x 128,
-# 128 x 128 and 128 x 64 in four; then 512 x 128 over four k ranges of unequal chunks
+@pytest.mark.parametrize("kernel,M,N,Kd,epilogue,S", GEMM_TILING_CASES)
+def test_gemm_every_tiling_exact_on_integer_grid(K, kernel, M, N, Kd, epilogue, S):
+    """Each tiling of the register-stationary and few-token kernels, by name, bit-exact where the arithmetic is exact, over
+    an output that held other values; split ranges reduced and as partials; the SwiGLU epilogue within 1e-3 of the oracle's
+    swiglu of the exact rows (its silu is fp32, rounded to fp16 twice) and equal to the swiglu kernel's where that takes
+    the shape."""
+    G = 128
+    assert K.gemm_kernel(M, N, Kd, G, epilogue, S) == kernel
+    packed, sz, wref = _grid_weights(N, Kd, G, seed=M + N + Kd)
+    x = torch.randint(-3, 4, (M, Kd), generator=gen(M + 1)).half()
+    want = torch.mm(x.to(DEV).double(), wref.to(DEV).double().t().contiguous()).half()     # exact sums, one rounding
+    if epilogue == 1:
+        act = torch.full((M, N // 2), 7.0, dtype=torch.half, device=DEV)
+        K.gemm_w4a16(packed, sz, x.to(DEV), act, G, epilogue=1)
+        assert_close(act, R.swiglu_ref(torch.cat([want[:, 0::2], want[:, 1::2]], 1).cpu()), 1e-3, kernel)
+        if N // 2 % 8 == 0:
+            sep = torch.empty_like(act)
+            for m in (0, M // 2, M - 1):
+                K.swiglu(torch.cat([want[m, 0::2], want[m, 1::2]]).contiguous(), sep[m])
+                assert torch.equal(act[m], sep[m]), (kernel, m)
+        return
+    need = K.gemm_workspace_bytes(M, N, Kd, G)
+    assert need == (S * M * N * 4 if S > 1 else 0)
+    ws = torch.full((need,), 0xFF, dtype=torch.uint8, device=DEV) if need else None
+    y = torch.full((M, N), 7.0, dtype=torch.half, device=DEV)
+    K.gemm_w4a16(packed, sz, x.to(DEV), y, G, workspace=ws)
+    assert torch.equal(y, want), kernel
+    if need:
+        ws.fill_(0xFF)
+        assert torch.equal(K.gemm_w4a16_parts(packed, sz, x.to(DEV), G, ws).double().sum(0).half(), want), kernel
+
+
+# more ragged M and N for whichever tiling the rule gives, from one chunk on, and four k ranges of unequal chunks
 @pytest.mark.parametrize("M,N,Kd,S", [(509, 25001, 256, 0), (1030, 5100, 256, 0), (500, 5003, 256, 0),
                                       (2000, 20002, 128, 0), (1500, 6140, 384, 0), (510, 4100, 128, 0),
                                       (1021, 4092, 14464, 4)])
@@ -406,9 +434,9 @@ def test_attention_prefill(K, D, n_q, n_kv, page, start, M):
                                              (128, 64, 32, 300, (1, 20))])
 def test_attention_prefill_rows_independent_of_batch(K, D, n_q, n_kv, M, ks):
     """A row's result does not depend on which other rows share its launch: the last rows of a prompt computed alone
-    (pos advanced, qkv sliced) are bit-identical to the same rows of the whole prompt. Both launches of a case have
-    grids on the same side of 256 workgroups (first case below, the others above), which sets the wave groups per
-    workgroup and with them the order in which a row's blocks are summed."""
+    (pos advanced, qkv sliced) are bit-identical to the same rows of the whole prompt. Both launches of a case take the
+    same workgroup shape (by their waves of 32 columns), which sets the groups that share a row's blocks and with them the
+    order in which those are summed."""
     page = 16
     kc, vc, bt = make_cache(M, n_kv, page, D=D, seed=11 + D)
     qkv = torch.randn(M, (n_q + 2 * n_kv) * D, generator=gen(12)).half()
@@ -553,7 +581,7 @@ def test_prefill_matches_oracle_and_teacher_force(K, D):
 def test_prefill_in_chunks_is_bit_exact(K):
     """Attention rows are computed independently of their batch, and for this model's shapes every chunk size takes
     the same GEMM configuration (64 x 64 tiles, four K groups; the configuration, and with it the fp32 summation order,
-    is chosen per M x N x K) and the same attention grid class (at most 256 workgroups): a prompt prefilled in three
+    is chosen per M x N x K) and the same attention workgroup shape (at most 512 waves of 32 columns): a prompt prefilled in three
     chunks leaves the same cache and logits as one pass."""
     m, _ = _model()
     prompt = _prompt(70, seed=2)
