@@ -84,15 +84,17 @@ __device__ __forceinline__ double partner(double v) {
   const float hi = partner<O>(__builtin_bit_cast(float, (uint32_t)(b >> 32)));
   return __builtin_bit_cast(double, (uint64_t)__builtin_bit_cast(uint32_t, hi) << 32 | __builtin_bit_cast(uint32_t, lo));
 }
-// over the WPG lanes of a group, from the farthest partner to the nearest
-template <int WPG>
+// over the WPG lanes of a group, from the nearest partner to the farthest: when lane ^ 4 is due the lanes of a quad hold the
+// same values, so lane ^ 7 serves (one instruction less: 1% of 4096 x 14336 without clip)
+template <int WPG, int O = 1>
 __device__ __forceinline__ void group_range(float& lo, float& hi) {
-  if constexpr (WPG > 1) {
-    lo = fminf(lo, partner<WPG / 2>(lo));
-    hi = fmaxf(hi, partner<WPG / 2>(hi));
-    group_range<WPG / 2>(lo, hi);
+  if constexpr (O < WPG) {
+    lo = fminf(lo, O == 4 ? DK_DPP_F32(lo, 0x141, 0xF) : partner<O>(lo));
+    hi = fmaxf(hi, O == 4 ? DK_DPP_F32(hi, 0x141, 0xF) : partner<O>(hi));
+    group_range<WPG, 2 * O>(lo, hi);
   }
 }
+// the same over sums, whose rounding depends on the order: from the farthest partner to the nearest
 template <int WPG>
 __device__ __forceinline__ void group_total(double& e) {
   if constexpr (WPG > 1) {
