@@ -363,7 +363,7 @@ gemm_w4a16_wide(const uint32_t* W, const uint32_t* SZ, const f16* X, f16* Y, int
 // lane l = 32 h + r of row tile i loads words 8h .. 8h+7 of row 32 i + r in the 128-wide k chunk (two 16-byte
 // loads) -- and are dequantized there, already in the MFMA A layout: no weight passes through LDS and each is
 // dequantized once. Only the token tile X [BM x 128] is staged in LDS (rows of 256 bytes, 16-byte chunk q of row t at
-// q ^ (t & 15)), written once per chunk and read by all four waves.
+// q ^ (t & 15)), written once per chunk and read by all the workgroup's waves.
 //   MFMA: v_mfma_f32_32x32x16_f16. A stream of independent 32x32x16 MFMAs runs at one per 32 clocks per SIMD (the
 //   dense fp16 rate), a stream of 16x16x32 ones at about three quarters of that, so the 32 x 32 form carries the
 //   kernel; the dequant's vector instructions issue between the MFMAs, one k step ahead of them. k order: in k step s (0..7) of a chunk, lane (h, r) takes word 8h + s of its row
@@ -803,15 +803,21 @@ bool rs_fills(int M, int N, int K, int log2G) {
 
 // Split-K (a workspace given, epilogue 0 or 2 = the partials alone): the k ranges S, 1 if the shape does not split. The
 // partials cost traffic (S x M x N x 4 bytes, written and read back) and, unless the next norm sums them, a launch.
-//   * M >= 768 and the unsplit kernel has its tiles: the S in 1, 2, 4 (16 chunks of 128 per range at least) of the least time
-//     over its best tiling, the partials priced at half of what a reduce launch reads them in (7 TB/s: most readers are
-//     norms that read them anyway); no split unless 5% better, nor where K is under 64 chunks. 4096 x 14336 at M 2048 228 us unsplit (256 x 128) against 298 split 2 ways over
-//     256 x 64 tiles of four waves, at M 1024 122 split 4 ways over 512 x 128 (125 split 2 ways over 256 x 128) against 148.
+//   * M >= 768 and the unsplit kernel has its tiles: the S in 1, 2, 4 (16 chunks of 128 per range at least) of the
+//     least time over its best tiling, the partials priced at half of what a reduce launch reads them in (7 TB/s: most
+//     readers are norms that read them anyway); no split unless 5% better, nor where K is under 64 chunks. 4096 x
+//     14336 at M 2048 228 us unsplit (256 x 128) against 298 split 2 ways over 256 x 64 tiles of four waves, at M 1024
+//     122 split 4 ways over 512 x 128 (125 split 2 ways over 256 x 128) against 148. Where K is long below 768 the
+//     next rule stands: at 4096 x 14336 the two agree within 1% up to there (M 656 S 4 101 us, S 2 102; M 759 S 2 101,
+//     S 4 102). It also splits rows that fill the CUs by themselves (28672 x 8192 at M 512 over 2 ranges: 238 us
+//     predicted, unsplit 213).
 //   * otherwise, when the unsplit kernel lacks its tiles or K has 64 chunks, the smallest power of two that gives 384
-//     workgroups of 256 x 64 (else 128 x 64) while every range keeps 16 chunks, if that reaches 192 (4096 x 14336 at M 512:
-//     S 4; 768 x 4096 at M 1600, 150 tiles, S 2: 25.8 us against 46.0 unsplit on the wide kernel; 256 x 16384 at M 768 20.9
-//     at S 8 against 30.7 at S 4; from M 768 on as many of 4 ranges as keep 16 chunks where even that does not reach 192:
-//     768 x 4096 at M 900 S 2 19.2 against 24.3 unsplit, 304 x 13312 at M 884 S 4 27.7 against 67.2; TinyLlama's qkv 2560 x 2048 at S 4, 4 chunks per range: 27 us against 19 unsplit).
+//     workgroups of 256 x 64 (else 128 x 64; so counted whatever tiling is then the fastest over S ranges) while every
+//     range keeps 16 chunks, if that reaches 192 (4096 x 14336 at M 512: S 4; 768 x 4096 at M 1600, 150 tiles, S 2:
+//     25.8 us against 46.0 unsplit on the wide kernel; 256 x 16384 at M 768 20.9 at S 8 against 30.7 at S 4; from M
+//     768 on as many of 4 ranges as keep 16 chunks where even that does not reach 192: 768 x 4096 at M 900 S 2 19.2
+//     against 24.3 unsplit, 304 x 13312 at M 884 S 4 27.7 against 67.2; TinyLlama's qkv 2560 x 2048 at S 4, 4 chunks
+//     per range: 27 us against 19 unsplit).
 //   * up to 128 tokens the partials are small and the alternative is the wide kernel with a few tiles, so there shorter
 //     ranges (5 chunks) pay while the 128 x 64 tiles alone leave three quarters of the CUs idle: 4096 x 14336 at M 64 20.8 us
 //     against 66.2, 4096 x 4096 at M 33 / 64 / 128 13.0 / 13.6 / 16.3 against 18.9 / 20.5 / 19.9, 2048 x 5632 at 64
